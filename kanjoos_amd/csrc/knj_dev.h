@@ -67,9 +67,12 @@ constexpr int kDppHalfMirror = 0x141; // lane i <- 7 - i within 8
 constexpr int kDppMirror = 0x140;     // lane i <- 15 - i within 16
 constexpr int kDppRor8 = 0x128;       // lane i <- (i + 8) % 16 within 16, i.e. i ^ 8
 
+// (every lane of these controls has a source, so the old value and the bound
+// control never show; this form of them lets the compiler fold the move into
+// the instruction that uses it)
 template <int CTRL>
 __device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
-  return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, 0xF, 0xF, false);
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, true);
 }
 
 // the value of lane l ^ 16
@@ -78,6 +81,17 @@ __device__ __forceinline__ uint32_t xor16_u32(uint32_t v) {
   // second result the odd rows
   const auto p = __builtin_amdgcn_permlane16_swap(v, v, false, false);
   return (__lane_id() & 16) ? p[0] : p[1];
+}
+
+// v of lane l and of lane l ^ 16 (or l ^ 32), in some order: all that a
+// commutative combination of the two needs
+__device__ __forceinline__ float2 pair16_f(float v) {
+  const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return make_float2(__uint_as_float(p[0]), __uint_as_float(p[1]));
+}
+__device__ __forceinline__ float2 pair32_f(float v) {
+  const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return make_float2(__uint_as_float(p[0]), __uint_as_float(p[1]));
 }
 
 // the value of lane l ^ 32
@@ -101,8 +115,14 @@ __device__ __forceinline__ float group_reduce(float v, Op op) {
   if constexpr (W >= 4) v = op(v, dpp_f<kDppXor2>(v));
   if constexpr (W >= 8) v = op(v, dpp_f<kDppHalfMirror>(v));
   if constexpr (W >= 16) v = op(v, dpp_f<kDppMirror>(v));
-  if constexpr (W >= 32) v = op(v, xor16_f(v));
-  if constexpr (W >= 64) v = op(v, xor32_f(v));
+  if constexpr (W >= 32) {
+    const float2 p = pair16_f(v);
+    v = op(p.x, p.y);
+  }
+  if constexpr (W >= 64) {
+    const float2 p = pair32_f(v);
+    v = op(p.x, p.y);
+  }
   return v;
 }
 
