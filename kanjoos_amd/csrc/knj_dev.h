@@ -439,21 +439,24 @@ __device__ __forceinline__ float q6k_quarter(const uint8_t* __restrict__ blk, in
 // 128 hf + 32 t + 8 o + i (t, i < 4, 8): ql bytes 64 hf + 8 o (quarters 0, 2)
 // and 64 hf + 32 + 8 o (quarters 1, 3), qh bytes 32 hf + 8 o, the scales of
 // sub-group o/2 of each quarter and d (dequant_q6_k, dequant.cpp:164-191).
-// Q6_K blocks are 210 bytes, so these runs are only 2-byte aligned: each is
-// read as three aligned words and shifted into place.
+// Q6_K blocks are 210 bytes, so these runs are only 2-byte aligned.
 struct Q6Unit {
   uint32_t l0a, l0b, l1a, l1b, ha, hb;  // ql run 0, ql run 1, qh run (8 bytes each)
-  int32_t sc[4];                        // the quarters' scales
+  uint32_t sa, sb, sh;                  // the half's 8 scales; quarter t's is byte 2 t + sh / 8
   uint32_t d;                           // f16 bits of d
+  __device__ __forceinline__ float scale(int t) const {
+    return (float)(int8_t)(((t & 2) ? sb : sa) >> (16 * (t & 1) + sh));
+  }
 };
 
+// Eight bytes at a 2-byte aligned address by one load (the device runs with
+// unaligned access on, as the compiler assumes; three aligned words shifted
+// into place are three loads and eight vector instructions).
 __device__ __forceinline__ void ld8_u2(const uint8_t* p, uint32_t& a, uint32_t& b) {
-  const uintptr_t addr = reinterpret_cast<uintptr_t>(p);
-  const uint32_t* w = reinterpret_cast<const uint32_t*>(addr & ~(uintptr_t)3);
-  const uint32_t w0 = w[0], w1 = w[1], w2 = w[2];
-  const uint32_t sh = (uint32_t)(addr & 3) * 8;
-  a = sh ? __builtin_amdgcn_alignbit(w1, w0, sh) : w0;
-  b = sh ? __builtin_amdgcn_alignbit(w2, w1, sh) : w1;
+  uint2 v;
+  __builtin_memcpy(&v, p, 8);
+  a = v.x;
+  b = v.y;
 }
 
 __device__ __forceinline__ Q6Unit q6_unit_load(const uint8_t* __restrict__ blk, int hf, int o) {
@@ -461,10 +464,8 @@ __device__ __forceinline__ Q6Unit q6_unit_load(const uint8_t* __restrict__ blk, 
   ld8_u2(blk + KNJ_Q6K_QL + 64 * hf + 8 * o, u.l0a, u.l0b);
   ld8_u2(blk + KNJ_Q6K_QL + 64 * hf + 32 + 8 * o, u.l1a, u.l1b);
   ld8_u2(blk + KNJ_Q6K_QH + 32 * hf + 8 * o, u.ha, u.hb);
-  // (scales and d by narrow loads, which stay inside the block)
-  const int8_t* sp = reinterpret_cast<const int8_t*>(blk + KNJ_Q6K_SC + 8 * hf + (o >> 1));
-#pragma unroll
-  for (int t = 0; t < 4; ++t) u.sc[t] = sp[2 * t];
+  ld8_u2(blk + KNJ_Q6K_SC + 8 * hf, u.sa, u.sb);
+  u.sh = 8 * (o >> 1);
   u.d = *reinterpret_cast<const uint16_t*>(blk + KNJ_Q6K_D);
   return u;
 }
@@ -489,7 +490,7 @@ __device__ __forceinline__ float q6_unit_dot(const Q6Unit& u, const float4 (&x8)
     acc += (float)((qb >> 8) & 0xFFu) * x8[t][1].y;
     acc += (float)((qb >> 16) & 0xFFu) * x8[t][1].z;
     acc += (float)(qb >> 24) * x8[t][1].w;
-    r += (float)u.sc[t] * (acc - 32.0f * sx[t]);
+    r += u.scale(t) * (acc - 32.0f * sx[t]);
   }
   return h2f(u.d) * r;
 }

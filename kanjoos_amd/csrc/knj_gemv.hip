@@ -205,71 +205,123 @@ __global__ __launch_bounds__(kBlock) void k_gemv_q4k_wide(const uint8_t* __restr
   }
 }
 
-// Q6_K rows of n_in <= 2048 (at most 64 units of 32 weights): lane = unit, so
-// every lane's x (32 values and 4 run sums) is the same for every row and
-// stays in registers; RS rows per wave step, all their loads issued first;
+// Q6_K rows of n_in <= 4096: LPR lanes per row, each with 64 weights of one
+// super-block: half hf, 16-run o of its four quarters (weights 128 hf + 32 t +
+// 16 o + i, t < 4, i < 16), which share one scale per quarter.  The lane's x
+// (64 values and 4 run sums) is the same for every row and stays in registers;
 // rows walked grid-stride (the argmax variant keeps the grid <= kMaxKeys).
-template <int RS>
-__global__ __launch_bounds__(kBlock) void k_gemv_q6k_u(const uint8_t* __restrict__ w, int n_in,
+// A lane reads its codes as three 16-byte pieces at 2-byte aligned addresses.
+// Bound by the vector memory unit and the vector instructions together.  With
+// 32 weights per lane, in 8-byte pieces (each as three aligned words), a row
+// took 14 loads of about 20 vector cache accesses and 4.9 vector instructions
+// a weight; now 5 loads serve two rows and 3.1 instructions a weight: the
+// 151,936 x 2048 head 60.5 -> 47.5 us (4.2 -> 5.4 TB/s).  Also measured there:
+// two and four rows per lane in flight 50.0 and 55.0 us, rows fetched into LDS
+// by DMA and decoded from there 76 us.
+struct Q6Run {
+  uint4 l0, l1, h;   // ql bytes of quarters 0 and 2, of 1 and 3, qh bytes
+  uint32_t sa, sb;   // the half's 8 scales; quarter t's is byte 2 t + o
+  uint32_t d;        // f16 bits of d
+};
+
+__device__ __forceinline__ Q6Run q6_run_load(const uint8_t* __restrict__ blk, int hf, int o) {
+  Q6Run r;
+  __builtin_memcpy(&r.l0, blk + KNJ_Q6K_QL + 64 * hf + 16 * o, 16);
+  __builtin_memcpy(&r.l1, blk + KNJ_Q6K_QL + 64 * hf + 32 + 16 * o, 16);
+  __builtin_memcpy(&r.h, blk + KNJ_Q6K_QH + 32 * hf + 16 * o, 16);
+  ld8_u2(blk + KNJ_Q6K_SC + 8 * hf, r.sa, r.sb);
+  r.d = *reinterpret_cast<const uint16_t*>(blk + KNJ_Q6K_D);
+  return r;
+}
+
+// sum over the run's 64 weights of w*x = d * sum_t sc_t * (sum_i q x - 32 sum_i x)
+__device__ __forceinline__ float q6_run_dot(const Q6Run& r, int o, const float (&x)[4][16], const float (&sx)[4]) {
+  const uint32_t sh = 8 * o;
+  float sum = 0.0f;
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const uint4 l = (t & 1) ? r.l1 : r.l0;
+    const uint32_t lw[4] = {l.x, l.y, l.z, l.w}, hw[4] = {r.h.x, r.h.y, r.h.z, r.h.w};
+    float a4[4] = {};  // (short chains: four of four terms)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const uint32_t q = ((lw[k] >> (4 * (t >> 1))) & 0x0F0F0F0Fu) | (((hw[k] >> (2 * t)) & 0x03030303u) << 4);
+      a4[k] += (float)(q & 0xFFu) * x[t][4 * k];
+      a4[k] += (float)((q >> 8) & 0xFFu) * x[t][4 * k + 1];
+      a4[k] += (float)((q >> 16) & 0xFFu) * x[t][4 * k + 2];
+      a4[k] += (float)(q >> 24) * x[t][4 * k + 3];
+    }
+    const float acc = (a4[0] + a4[1]) + (a4[2] + a4[3]);
+    const float sc = (float)(int8_t)(((t & 2) ? r.sb : r.sa) >> (16 * (t & 1) + sh));
+    sum += sc * (acc - 32.0f * sx[t]);
+  }
+  return h2f(r.d) * sum;
+}
+
+template <int LPR>
+__global__ __launch_bounds__(kBlock, 4) void k_gemv_q6k_u(const uint8_t* __restrict__ w, int n_in,
                                                        int n_out, const float* __restrict__ x,
                                                        const float* __restrict__ nw, float eps,
                                                        const float* __restrict__ resid,
                                                        float* __restrict__ y,
                                                        unsigned long long* argmax) {
-  __shared__ float xs[xpad_size(2048)];
-  __shared__ float xs8[256];
+  __shared__ float xs[xpad_size(4096)];
+  __shared__ float xs16[256];
   __shared__ float red[8];
+  constexpr int RPW = 64 / LPR;  // rows of a row-step
   stage_x(x, nw, eps, n_in, xs, red);
-  for (int g = threadIdx.x; 8 * g < n_in; g += kBlock) {
-    const float4 a = *reinterpret_cast<const float4*>(xs + xpad(8 * g));
-    const float4 b = *reinterpret_cast<const float4*>(xs + xpad(8 * g) + 4);
-    xs8[g] = ((a.x + a.y) + (a.z + a.w)) + ((b.x + b.y) + (b.z + b.w));
+  for (int g = threadIdx.x; 16 * g < n_in; g += kBlock) {
+    float s = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const float4 a = *reinterpret_cast<const float4*>(xs + xpad(16 * g) + 4 * k);
+      s += (a.x + a.y) + (a.z + a.w);
+    }
+    xs16[g] = s;
   }
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int nb = n_in / KNJ_QK, nunits = 8 * nb;
-  const bool active = lane < nunits;
-  const int u = active ? lane : 0;
-  const int b = u >> 3, hf = (u >> 2) & 1, o = u & 3;
-  float4 x8[4][2];
-  float sx[4];
+  const int sub = lane % LPR, rsub = lane / LPR;
+  const int nb = n_in / KNJ_QK;
+  const bool active = sub < 4 * nb;
+  const int u = active ? sub : 0, b = u >> 2, hf = (u >> 1) & 1, o = u & 1;
+  float xv[4][16], sx[4];
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
-    const int i = 256 * b + 128 * hf + 32 * t + 8 * o;
-    x8[t][0] = *reinterpret_cast<const float4*>(xs + xpad(i));
-    x8[t][1] = *reinterpret_cast<const float4*>(xs + xpad(i) + 4);
-    sx[t] = xs8[i >> 3];
+    const int i = 256 * b + 128 * hf + 32 * t + 16 * o;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const float4 a = *reinterpret_cast<const float4*>(xs + xpad(i) + 4 * k);
+      xv[t][4 * k] = a.x;
+      xv[t][4 * k + 1] = a.y;
+      xv[t][4 * k + 2] = a.z;
+      xv[t][4 * k + 3] = a.w;
+    }
+    sx[t] = xs16[i >> 4];
   }
   const uint64_t rb = (uint64_t)nb * KNJ_Q6K_BLOCK;
   const uint8_t* wu = w + (uint64_t)b * KNJ_Q6K_BLOCK;
   unsigned long long best = 0;
-  const int stride = gridDim.x * (kBlock / 64) * RS;
-  for (int r0 = (blockIdx.x * (kBlock / 64) + wave) * RS; r0 < n_out; r0 += stride) {
-    Q6Unit q[RS];
-#pragma unroll
-    for (int st = 0; st < RS; ++st) q[st] = q6_unit_load(wu + (uint64_t)min(r0 + st, n_out - 1) * rb, hf, o);
-    float rv[RS];
-#pragma unroll
-    for (int st = 0; st < RS; ++st) rv[st] = resid ? resid[min(r0 + st, n_out - 1)] : 0.0f;
-#pragma unroll
-    for (int st = 0; st < RS; ++st) {
-      const float acc = group_sum<64>(active ? q6_unit_dot(q[st], x8, sx) : 0.0f);
-      const int row = r0 + st;
-      if (lane == 0 && row < n_out) {
-        const float v = resid ? rv[st] + acc : acc;
-        y[row] = v;
-        if (argmax) {
-          const unsigned long long k = argmax_key(v, row);
-          best = k > best ? k : best;
-        }
+  const int stride = gridDim.x * (kBlock / 64) * RPW;
+  for (int r0 = (blockIdx.x * (kBlock / 64) + wave) * RPW; r0 < n_out; r0 += stride) {
+    const int row = r0 + rsub, rc = min(row, n_out - 1);
+    const Q6Run q = q6_run_load(wu + (uint64_t)rc * rb, hf, o);
+    const float rv = resid ? resid[rc] : 0.0f;
+    const float acc = group_sum<LPR>(active ? q6_run_dot(q, o, xv, sx) : 0.0f);
+    if (sub == 0 && row < n_out) {
+      const float v = resid ? rv + acc : acc;
+      y[row] = v;
+      if (argmax) {
+        const unsigned long long k = argmax_key(v, row);
+        best = k > best ? k : best;
       }
     }
   }
   if (argmax) block_argmax_store(best, argmax);
 }
 
-// Q6_K rows: 8 quarters per block, LPR lanes per row, activations in LDS.
-template <int LPR>
+// Q6_K rows of n_in > 4096: 8 quarters per block, a wave per row, activations
+// in LDS.
 __global__ __launch_bounds__(kBlock) void k_gemv_q6k(const uint8_t* __restrict__ w, int n_in,
                                                      int n_out, const float* __restrict__ x,
                                                      const float* __restrict__ nw, float eps,
@@ -301,23 +353,18 @@ __global__ __launch_bounds__(kBlock) void k_gemv_q6k(const uint8_t* __restrict__
   const int nb = n_in / KNJ_QK, nq = 8 * nb;
   const uint64_t rb = (uint64_t)nb * KNJ_Q6K_BLOCK;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int sub = lane % LPR, rsub = lane / LPR;
-  constexpr int RPW = 64 / LPR;
-  const int stride = gridDim.x * (kBlock / 64) * RPW;
+  const int stride = gridDim.x * (kBlock / 64);
   unsigned long long best = 0;
-  for (int row0 = (blockIdx.x * (kBlock / 64) + wave) * RPW; row0 < n_out; row0 += stride) {
-    const int row = row0 + rsub;
+  for (int row = blockIdx.x * (kBlock / 64) + wave; row < n_out; row += stride) {
     float acc = 0.0f;
-    if (row < n_out) {
-      const uint8_t* rp = w + (uint64_t)row * rb;
-      for (int s = sub; s < nq; s += LPR) {
-        const int bb = s >> 3;
-        acc += q6k_quarter(rp + (uint64_t)bb * KNJ_Q6K_BLOCK, (s >> 2) & 1, s & 3,
-                           xsq + bb * KNJ_QK + 128 * ((s >> 2) & 1) + 32 * (s & 3));
-      }
+    const uint8_t* rp = w + (uint64_t)row * rb;
+    for (int s = lane; s < nq; s += 64) {
+      const int bb = s >> 3;
+      acc += q6k_quarter(rp + (uint64_t)bb * KNJ_Q6K_BLOCK, (s >> 2) & 1, s & 3,
+                         xsq + bb * KNJ_QK + 128 * ((s >> 2) & 1) + 32 * (s & 3));
     }
-    acc = group_sum<LPR>(acc);
-    if (sub == 0 && row < n_out) {
+    acc = group_sum<64>(acc);
+    if (lane == 0) {
       const float v = resid ? resid[row] + acc : acc;
       y[row] = v;
       if (argmax) {
@@ -541,14 +588,11 @@ bool bf16_fast(int n_in) {
 
 // Grids of the argmax-capable GEMVs (Q6_K, BF16, F32); one key per workgroup.
 int gemv_grid(int type, int n_in, int n_out) {
-  if (type == KNJ_TYPE_Q6_K && n_in <= 2048) {
-    constexpr int RS = 4;
-    return std::max(1, std::min(2048, (n_out + 4 * RS - 1) / (4 * RS)));
-  }
-  if (type == KNJ_TYPE_Q6_K) {
-    const int lpr = std::min(64, pow2_at_least(8 * (n_in / KNJ_QK)));
-    const int rows_per_block = 4 * (64 / lpr);
-    return std::max(1, std::min(kMaxKeys, (n_out + rows_per_block - 1) / rows_per_block));
+  if (type == KNJ_TYPE_Q6_K && n_in <= 4096) {
+    // three workgroups per CU, the rows walked grid-stride (the 151,936-row
+    // head: 52.4 us at 512, 47.5 at 768, 54.3 at 1024, 53.3 at 2048)
+    const int rows = 4 * (64 / pow2_at_least(n_in / 64));  // of a workgroup's step
+    return std::max(1, std::min(768, (n_out + rows - 1) / rows));
   }
   if (type == KNJ_TYPE_BF16 && bf16_fast(n_in)) {
     // two rows per wave step, up to kMaxKeys workgroups: the 151,936-row
@@ -586,24 +630,23 @@ hipError_t launch_gemv(const GemvArgs& a, hipStream_t s) {
                        a.norm_w, a.eps, a.resid, a.y);
     return hipGetLastError();
   }
-  if (a.type == KNJ_TYPE_Q6_K && a.n_in <= 2048) {
-    KNJ_LAUNCH(k_gemv_q6k_u<4>, dim3(gemv_grid(a.type, a.n_in, a.n_out)), dim3(kBlock), 0, s,
-                       a.w, a.n_in, a.n_out, a.x, a.norm_w, a.eps, a.resid, a.y, a.argmax_key);
-    return hipGetLastError();
+  if (a.type == KNJ_TYPE_Q6_K && a.n_in <= 4096) {
+    const dim3 grid(gemv_grid(a.type, a.n_in, a.n_out));
+    const int lpr = pow2_at_least(a.n_in / 64);
+#define G6U(L)                                                                                     \
+  if (lpr == L) {                                                                                  \
+    KNJ_LAUNCH(k_gemv_q6k_u<L>, grid, dim3(kBlock), 0, s, a.w, a.n_in, a.n_out, a.x,               \
+               a.norm_w, a.eps, a.resid, a.y, a.argmax_key);                                       \
+    return hipGetLastError();                                                                      \
+  }
+    G6U(4) G6U(8) G6U(16) G6U(32) G6U(64)
+#undef G6U
+    return hipErrorInvalidValue;
   }
   if (a.type == KNJ_TYPE_Q6_K) {
-    const int lpr = std::min(64, pow2_at_least(8 * (a.n_in / KNJ_QK)));
-    const size_t lds = (size_t)a.n_in * 4;
-    const int grid = gemv_grid(a.type, a.n_in, a.n_out);
-#define G6(L)                                                                                 \
-  if (lpr == L) {                                                                             \
-    KNJ_LAUNCH(k_gemv_q6k<L>, dim3(grid), dim3(kBlock), lds, s, a.w, a.n_in, a.n_out, \
-                       a.x, a.norm_w, a.eps, a.resid, a.y, a.argmax_key);                     \
-    return hipGetLastError();                                                                 \
-  }
-    G6(8) G6(16) G6(32) G6(64)
-#undef G6
-    return hipErrorInvalidValue;
+    KNJ_LAUNCH(k_gemv_q6k, dim3(gemv_grid(a.type, a.n_in, a.n_out)), dim3(kBlock), (size_t)a.n_in * 4, s,
+               a.w, a.n_in, a.n_out, a.x, a.norm_w, a.eps, a.resid, a.y, a.argmax_key);
+    return hipGetLastError();
   }
   if (a.type == KNJ_TYPE_BF16 && bf16_fast(a.n_in)) {
     const int nj = a.n_in / 512;

@@ -961,8 +961,8 @@ __global__ __launch_bounds__(512) void k_expert_down8(ExpertArgs a) {
 // kernel; activations and their 8-element sums staged once per workgroup.
 // STAGED: the 8 rows of a wave's expert are one contiguous, 16-byte aligned
 // run (8 x 630 bytes at n_ff = 768), fetched with 16-byte loads into LDS and
-// decoded from there, instead of three unaligned 8-byte runs, four scale
-// bytes and d per 32-weight unit straight from memory.
+// decoded from there, instead of four unaligned 8-byte runs and d per
+// 32-weight unit straight from memory.
 constexpr int kQ6StageLoads = 7;  // 16-byte loads per lane: 8 rows of n_ff <= 1024
 
 // q6_unit_load from a Q6_K block at byte `blk` of an LDS region (2-byte
@@ -980,9 +980,8 @@ __device__ __forceinline__ Q6Unit q6_unit_load_lds(const uint8_t* region, uint32
   lds_ld8(w4, blk + KNJ_Q6K_QL + 64 * hf + 8 * o, u.l0a, u.l0b);
   lds_ld8(w4, blk + KNJ_Q6K_QL + 64 * hf + 32 + 8 * o, u.l1a, u.l1b);
   lds_ld8(w4, blk + KNJ_Q6K_QH + 32 * hf + 8 * o, u.ha, u.hb);
-  const int8_t* sp = reinterpret_cast<const int8_t*>(region + blk + KNJ_Q6K_SC + 8 * hf + (o >> 1));
-#pragma unroll
-  for (int t = 0; t < 4; ++t) u.sc[t] = sp[2 * t];
+  lds_ld8(w4, blk + KNJ_Q6K_SC + 8 * hf, u.sa, u.sb);
+  u.sh = 8 * (o >> 1);
   u.d = *reinterpret_cast<const uint16_t*>(region + blk + KNJ_Q6K_D);
   return u;
 }
