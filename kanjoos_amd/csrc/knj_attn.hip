@@ -175,8 +175,15 @@ constexpr int kLdsOnly = vm_lds_imm(63);
 // chunk and zeroes the V rows past it (slots past the valid length under a
 // weight of 0).  The query/key/value, norm and RoPE loads are issued before
 // the first chunk's DMA (measured 1-3% faster per step than the chunk first).
-template <int D>
-__global__ __launch_bounds__(kBlock, 4) void k_attention(AttnArgs a, int cpw) {  // 4 waves per SIMD: 128 VGPRs
+// With a RopeRow the step's RoPE row and position are kernel arguments (a
+// caller that holds them on the host needs no copy to the device); the row is
+// read by vector loads from the argument segment, where the argument lies at
+// the next 16-byte boundary behind the two before it.
+constexpr size_t kRopeRowOffset = (sizeof(AttnArgs) + sizeof(int) + 15) & ~(size_t)15;
+static_assert(alignof(RopeRow) == 16, "kernel argument layout");
+
+template <int D, class... Row>
+__global__ __launch_bounds__(kBlock, 4) void k_attention(AttnArgs a, int cpw, Row... row) {  // 4 waves per SIMD: 128 VGPRs
   constexpr int ROWH = D + 8;            // f16 elements per query LDS row (16-byte pad)
   constexpr int EROW = kChunk + 4;       // floats per score row
   constexpr int T = D / 4;               // threads per head for the q pass
@@ -205,8 +212,15 @@ __global__ __launch_bounds__(kBlock, 4) void k_attention(AttnArgs a, int cpw) { 
   const float* qz = a.q + z * a.qkv_stride;
   const float* kz = a.k + z * a.qkv_stride;
   const float* vz = a.v + z * a.qkv_stride;
-  const float* rc = a.rope_cos + (uint64_t)z * a.rope_stride;
-  const float* rs = a.rope_sin + (uint64_t)z * a.rope_stride;
+  const float *rc, *rs;
+  if constexpr (sizeof...(Row) != 0) {
+    rc = (const float*)((const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr() +
+                        kRopeRowOffset);
+    rs = rc + D / 2;
+  } else {
+    rc = a.rope_cos + (uint64_t)z * a.rope_stride;
+    rs = a.rope_sin + (uint64_t)z * a.rope_stride;
+  }
   const uint64_t hstride = (uint64_t)n_split * (D + 2);
   // wave w's DMA instruction i fills bytes (w NI + i) KB .. +1 KB of the
   // chunk's K and V (rows past the cache clamp to its last row)
@@ -241,7 +255,10 @@ __global__ __launch_bounds__(kBlock, 4) void k_attention(AttnArgs a, int cpw) { 
   // the position by a scalar load (asm: as a vector load, the compiler's wait
   // for it would also wait for the DMA issued before it)
   int pos;
-  asm volatile("s_load_dword %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=s"(pos) : "s"(a.pos + z) : "memory");
+  if constexpr (sizeof...(Row) != 0)
+    pos = (row.pos, ...);
+  else
+    asm volatile("s_load_dword %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=s"(pos) : "s"(a.pos + z) : "memory");
   vm_wait7<2 * NI>(l_q, l_qn, l_k, l_v, l_kn, l_cs, l_sn);
   const float4 qraw = as_f4(l_q), qnw = as_f4(l_qn), kraw = as_f4(l_k), vraw = as_f4(l_v);
   const float4 knw = as_f4(l_kn), cs = as_f4(l_cs), sn = as_f4(l_sn);
@@ -902,10 +919,11 @@ int attn_splits(int n_ctx) { return (n_ctx + kChunk - 1) / kChunk; }
 // partition 2.55), up to kMaxSplit with several sequences (the per-head merge)
 constexpr int kMaxSplit = 256, kMaxSplit1 = 103;
 
-hipError_t launch_attention(const AttnArgs& a, hipStream_t s) {
+hipError_t launch_attention(const AttnArgs& a, hipStream_t s, const RopeRow* row) {
   // one 64-slot chunk per workgroup up to kMaxSplit chunks; beyond, several
   // chunks per workgroup so the merge sees at most kMaxSplit partials per head
-  const int chunks = attn_splits(a.n_ctx);
+  // (a position known here needs its own slots' chunks only)
+  const int chunks = attn_splits(row ? row->pos + 1 : a.n_ctx);
   // several sequences fill the chip with their own splits: at least three
   // chunks per workgroup there (measured at 32 sequences x 2048 slots: 8.55
   // ms/step with two, 8.42 with three, 8.59 with four; one chunk is faster at
@@ -915,8 +933,12 @@ hipError_t launch_attention(const AttnArgs& a, hipStream_t s) {
   const int n_split = (chunks + cpw - 1) / cpw;
   if (n_split > max_split) return hipErrorInvalidValue;
   const int z = std::max(1, a.n_seq);
+  if (row && (z != 1 || row->pos < 0 || row->pos >= a.n_ctx)) return hipErrorInvalidValue;
   if (a.head_dim == 128) {
-    KNJ_LAUNCH(k_attention<128>, dim3(a.n_head_kv, n_split, z), dim3(kBlock), 0, s, a, cpw);
+    if (row)
+      KNJ_LAUNCH((k_attention<128, RopeRow>), dim3(a.n_head_kv, n_split, z), dim3(kBlock), 0, s, a, cpw, *row);
+    else
+      KNJ_LAUNCH(k_attention<128>, dim3(a.n_head_kv, n_split, z), dim3(kBlock), 0, s, a, cpw);
     // up to 128 splits: 16 dims per workgroup, 16 parts of at most 8 splits
     // (the loads a part holds cost at short contexts)
     if (z == 1 && !a.split_hi && n_split <= 128)
@@ -926,7 +948,10 @@ hipError_t launch_attention(const AttnArgs& a, hipStream_t s) {
     else
       KNJ_LAUNCH(k_attn_merge_head<128>, dim3(a.n_head, z), dim3(kBlock), 0, s, a, n_split);
   } else if (a.head_dim == 64) {
-    KNJ_LAUNCH(k_attention<64>, dim3(a.n_head_kv, n_split, z), dim3(kBlock), 0, s, a, cpw);
+    if (row)
+      KNJ_LAUNCH((k_attention<64, RopeRow>), dim3(a.n_head_kv, n_split, z), dim3(kBlock), 0, s, a, cpw, *row);
+    else
+      KNJ_LAUNCH(k_attention<64>, dim3(a.n_head_kv, n_split, z), dim3(kBlock), 0, s, a, cpw);
     if (z == 1 && !a.split_hi && n_split <= 128)
       KNJ_LAUNCH((k_attn_merge<64, 16, 32>), dim3(a.n_head * 2, z), dim3(kBlock), 0, s, a, n_split);
     else if (z == 1 && !a.split_hi && n_split <= 256)

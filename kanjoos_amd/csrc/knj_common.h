@@ -226,7 +226,13 @@ struct AttnArgs {
   _Float16 *split_hi = nullptr, *split_lo = nullptr, *split_shi = nullptr, *split_slo = nullptr;
 };
 int attn_splits(int n_ctx);
-hipError_t launch_attention(const AttnArgs& a, hipStream_t s);
+// A step's RoPE row (cos then sin, D/2 each) and position held by the host:
+// with one, rope_cos, rope_sin and pos of the arguments are not read.
+struct alignas(16) RopeRow {
+  float tab[128];
+  int pos;
+};
+hipError_t launch_attention(const AttnArgs& a, hipStream_t s, const RopeRow* row = nullptr);
 
 // Attention of a prompt chunk (Model::forward with n > 1,
 // /root/reference/src/model/model.cpp:560-616): rows t < n_rows at positions

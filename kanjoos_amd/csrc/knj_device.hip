@@ -404,25 +404,23 @@ int knj_attention_step(const float* q, const float* k, const float* v, const flo
   hipStream_t s = (hipStream_t)stream;
   // cos/sin of this position, computed like the model's table (model.cpp:227-230, 278-279)
   const int half = head_dim / 2;
-  std::vector<float> tab(2 * (size_t)half + 64);
+  RopeRow row;
   for (int i = 0; i < half; ++i) {
     const float inv = std::pow(rope_base, -2.0f * (float)i / (float)head_dim);
     const float th = (float)pos * inv;
-    tab[i] = std::cos(th);
-    tab[half + i] = std::sin(th);
+    row.tab[i] = std::cos(th);
+    row.tab[half + i] = std::sin(th);
   }
-  std::memcpy(&tab[2 * half], &pos, sizeof(int));
-  const int n_split = attn_splits(n_ctx);
-  const uint64_t part_bytes = (uint64_t)n_head * n_split * (head_dim + 2) * 4;
-  uint8_t* scr = (uint8_t*)device_scratch(1024 + part_bytes, s);
-  if (!scr) return hip_fail(hipErrorOutOfMemory, "scratch");
-  float* dtab = (float*)scr;
-  int* dpos = (int*)(scr + 2 * half * 4);
-  KNJ_HIP(hipMemcpyAsync(scr, tab.data(), 2 * half * 4 + 4, hipMemcpyHostToDevice, s));
-  AttnArgs a{q, k, v, q_norm, k_norm, eps, dtab, dtab + half, dpos, k_cache, v_cache, n_head, n_head_kv,
-             head_dim, n_ctx, 1.0f / std::sqrt((float)head_dim), (float*)(scr + 1024), out};
-  KNJ_HIP(launch_attention(a, s));
-  KNJ_HIP(hipStreamSynchronize(s));  // the host table must outlive the copy
+  row.pos = pos;
+  const uint64_t part_bytes = (uint64_t)n_head * attn_splits(n_ctx) * (head_dim + 2) * 4;
+  float* part = (float*)device_scratch(part_bytes, s);
+  if (!part) return hip_fail(hipErrorOutOfMemory, "scratch");
+  // (row and position go with the launch: 21.2 us a call at 4096 slots and 29.6
+  // at 32,768, copied to the device first 25.3 and 34.4)
+  AttnArgs a{q, k, v, q_norm, k_norm, eps, nullptr, nullptr, nullptr, k_cache, v_cache, n_head, n_head_kv,
+             head_dim, n_ctx, 1.0f / std::sqrt((float)head_dim), part, out};
+  KNJ_HIP(launch_attention(a, s, &row));
+  KNJ_HIP(hipStreamSynchronize(s));  // the call returns with its output written
   return KNJ_OK;
 }
 
