@@ -1145,62 +1145,107 @@ __device__ __forceinline__ bf16x8 ld_b8(const uint16_t* p) {
 }
 
 // out[p][row] = W[row] . x_p for bf16 W [n_out][n_in] and tiles of 32 pairs
-// (blockIdx.y = tile): workgroup = 128 rows, wave = 32, lane l owns row l % 32;
-// three 32x32x16 bf16 matrix-core steps per 16 weights (x hi, mid, lo).
-__global__ __launch_bounds__(kBlock) void k_dense_bf16(const uint16_t* __restrict__ w, int n_in,
-                                                       int n_out, int P,
-                                                       const uint16_t* __restrict__ xh,
-                                                       const uint16_t* __restrict__ xm,
-                                                       const uint16_t* __restrict__ xl,
-                                                       float* __restrict__ out) {
+// (blockIdx.y = tile): workgroup = 64 rows, wave w = the 64-weight steps w,
+// w + 4, ... of all of them (lane l owns rows l % 32 and 32 + l % 32); three
+// 32x32x16 bf16 matrix-core steps per 16 weights and 32 rows (x hi, mid, lo).
+// The four waves' sums meet in LDS.  Bound by the weights' bytes once enough of
+// them are in flight: 32 rows of 32,768 x 2048 took 70.6 us (1.9 TB/s) with a
+// workgroup of 128 rows, one wave per 32 rows and SIMD and no load ahead of
+// its use; 42.8 us (3.1 TB/s) with the K range over the waves, 64 rows per
+// activation load and a step of loads in flight.
+constexpr int kBfRows = 64;
+
+struct Bf16Step {
+  bf16x8 w[2][4], x[3][4];
+};
+
+__global__ __launch_bounds__(kBlock, 2) void k_dense_bf16(const uint16_t* __restrict__ w, int n_in,
+                                                          int n_out, int P,
+                                                          const uint16_t* __restrict__ xh,
+                                                          const uint16_t* __restrict__ xm,
+                                                          const uint16_t* __restrict__ xl,
+                                                          float* __restrict__ out) {
+  __shared__ float red[kBlock / 64][2][16][64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int rbase = blockIdx.x * kRowsWG + wave * 32;
-  if (rbase >= n_out) return;
-  const int row = min(rbase + (lane & 31), n_out - 1), kh = lane >> 5;
+  const int rbase = blockIdx.x * kBfRows, kh = lane >> 5;
   const int p0 = blockIdx.y * kTok, cnt = min(kTok, P - p0);
   const int pj = p0 + min(lane & 31, cnt - 1);
   const uint64_t qs = (uint64_t)P * 8;
-  const uint16_t* wr = w + (uint64_t)row * n_in + 8 * kh;
+  const uint16_t* w0 = w + (uint64_t)min(rbase + (lane & 31), n_out - 1) * n_in + 8 * kh;
+  const uint16_t* w1 = w + (uint64_t)min(rbase + 32 + (lane & 31), n_out - 1) * n_in + 8 * kh;
   const uint64_t xo = (uint64_t)pj * 8 + kh * qs;
-  f32x16 acc = {};
-  for (int k0 = 0; k0 < n_in; k0 += 64) {
-    bf16x8 b[4], ah[4], am[4], al[4];
+  auto load = [&](int st, Bf16Step& r) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      b[u] = ld_b8(wr + k0 + 16 * u);
-      const uint64_t q = (uint64_t)((k0 + 16 * u) / 8) * qs + xo;
-      ah[u] = ld_b8(xh + q);
-      am[u] = ld_b8(xm + q);
-      al[u] = ld_b8(xl + q);
+      r.w[0][u] = ld_b8(w0 + 64 * st + 16 * u);
+      r.w[1][u] = ld_b8(w1 + 64 * st + 16 * u);
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[u], b[u], acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(am[u], b[u], acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al[u], b[u], acc, 0, 0, 0);
+      const uint64_t q = (uint64_t)(8 * st + 2 * u) * qs + xo;
+      r.x[0][u] = ld_b8(xh + q);
+      r.x[1][u] = ld_b8(xm + q);
+      r.x[2][u] = ld_b8(xl + q);
+    }
+  };
+  f32x16 acc[2] = {};
+  const int steps = n_in / 64;
+  if (wave < steps) {
+    Bf16Step cur, nxt;
+    load(wave, cur);
+    for (int st = wave; st < steps; st += 4) {
+      load(st + 4 < steps ? st + 4 : st, nxt);
+      // the loads stay ahead of the products (the scheduler would sink each to
+      // its use: 90 VGPRs, nothing in flight)
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+          for (int t = 0; t < 2; ++t)
+            acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur.x[c][u], cur.w[t][u], acc[t], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      cur = nxt;
     }
   }
-  if (rbase + (lane & 31) >= n_out) return;
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) red[wave][t][i][lane] = acc[t][i];
+  __syncthreads();
+  // wave w: row tile w / 2, pairs' registers 8 (w % 2) ..
+  const int t = wave >> 1, row = rbase + 32 * t + (lane & 31);
+  if (row >= n_out) return;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const int i = 8 * (wave & 1) + q;
+    const float v = (red[0][t][i][lane] + red[1][t][i][lane]) + (red[2][t][i][lane] + red[3][t][i][lane]);
     const int tj = 8 * (i / 4) + 4 * kh + (i % 4);
-    if (tj < cnt) out[(uint64_t)(p0 + tj) * n_out + row] = acc[i];
+    if (tj < cnt) out[(uint64_t)(p0 + tj) * n_out + row] = v;
   }
 }
 
 // Greedy token of each row of logits [m][n] (first maximum wins), in two
-// passes: workgroup (c, r) reduces chunk c of 8192 entries of row r to one
-// packed (value, index) key; then one workgroup per row reduces its keys.
-constexpr int kArgChunk = 8192;
+// passes: workgroup (c, r) reduces chunk c of 2048 entries of row r to one
+// packed (value, index) key, all its loads issued together; then one workgroup
+// per row reduces its keys.  32 rows of 32,768: 4.7 us (a launch's time), 10
+// with chunks of 8192 read one entry after the other.
+constexpr int kArgChunk = 2048;
 
 __global__ __launch_bounds__(kBlock) void k_argmax_part(const float* __restrict__ logits, int n,
                                                         unsigned long long* __restrict__ keys) {
   const int r = blockIdx.y, c = blockIdx.x;
   const float* row = logits + (uint64_t)r * n;
   const int i0 = c * kArgChunk, i1 = min(n, i0 + kArgChunk);
+  float v[kArgChunk / kBlock];
+#pragma unroll
+  for (int u = 0; u < kArgChunk / kBlock; ++u) v[u] = row[min(i0 + (int)threadIdx.x + u * kBlock, i1 - 1)];
   unsigned long long best = 0;
-  for (int i = i0 + threadIdx.x; i < i1; i += kBlock) {
-    const unsigned long long k = argmax_key(row[i], i);
+#pragma unroll
+  for (int u = 0; u < kArgChunk / kBlock; ++u) {
+    // (a clamped lane repeats entry i1 - 1)
+    const unsigned long long k = argmax_key(v[u], min(i0 + (int)threadIdx.x + u * kBlock, i1 - 1));
     best = k > best ? k : best;
   }
   best = wave_max_u64(best);
@@ -1656,7 +1701,7 @@ hipError_t launch_dense_bf16(const uint16_t* w, int n_in, int n_out, int m, cons
   uint16_t* xm = (uint16_t*)take(P * n_in * 2);
   uint16_t* xl = (uint16_t*)take(P * n_in * 2);
   KNJ_LAUNCH(k_split_bf16x3, dim3(m), dim3(kBlock), 0, s, x, n_in, m, xh, xm, xl);
-  KNJ_LAUNCH(k_dense_bf16, dim3((n_out + kRowsWG - 1) / kRowsWG, (m + kTok - 1) / kTok),
+  KNJ_LAUNCH(k_dense_bf16, dim3((n_out + kBfRows - 1) / kBfRows, (m + kTok - 1) / kTok),
                      dim3(kBlock), 0, s, w, n_in, n_out, m, xh, xm, xl, out);
   return hipGetLastError();
 }

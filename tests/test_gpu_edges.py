@@ -44,3 +44,32 @@ def test_gemv_q6k_edges(device, n_in, n_out, fused):
     got = dy.download(np.float32).astype(np.float64)
     assert np.all(np.abs(got - want) <= bound)
     assert rel_rmse(got, want) <= 1e-5
+
+
+@pytest.mark.parametrize("n_embd,n_vocab,B", [(256, 65, 1), (512, 2049, 3), (1280, 4127, 33), (2048, 2048, 5)])
+def test_batch_bf16_head_edges(device, n_embd, n_vocab, B):
+    """The batched bf16 head and its argmax at ragged row counts (64-row
+    workgroups, 2048-entry argmax chunks), at one tile of sequences and more,
+    and at widths that leave the four K-splits uneven: logits against the
+    oracle's within the parity bar (1e-5), the greedy token exactly the batch's
+    own first maximum."""
+    print(f"batch head {n_embd}x{n_vocab} B={B}", flush=True)
+    cfg = dict(n_layer=1, n_embd=n_embd, n_head=8, n_head_kv=2, head_dim=64, n_ff=256, n_expert=16,
+               n_expert_used=4, n_vocab=n_vocab, n_ctx=64)
+    gm = K.Model.synthetic(K.qwen3_30b_a3b(**cfg), seed=SEED)
+    toks = (np.arange(B, dtype=np.int32) * 7 + 1) % n_vocab
+    img = gm.download_image()
+    batch = K.Batch(gm, B, 64)
+    lg = batch.forward(toks)
+    om = O.OracleModel(O.make_config(**cfg), seed=SEED, image=img)
+    for s in range(B):
+        om.reset()
+        om.set_kv_source(*batch.kv_download(s))  # the cache's f16 roundings are the device's
+        assert rel_rmse(lg[s], om.forward([int(toks[s])])) <= 1e-5, s
+    om.close()
+    batch.close()
+    batch = K.Batch(gm, B, 64)
+    first = batch.decode_greedy(toks, 1)
+    batch.close()
+    assert np.array_equal(np.asarray(first).reshape(-1), lg.argmax(axis=1))
+    gm.close()
