@@ -287,17 +287,16 @@ __global__ __launch_bounds__(kBlock) void k_route_batch(const float* __restrict_
 }
 
 // ------------------------------------------------------------------ bucketing
-// One workgroup: pairs (token, slot) grouped by expert.  offsets[e] is the
-// first pair of expert e (offsets[E] = m*k); pair_tok[q] the token of pair q;
-// pair_of[t*k + s] the pair of token t's slot s; items the (expert, first
-// pair) of every tile of `tile` pairs.  The order of pairs within an expert does
+// One workgroup: pairs (token, slot) grouped by expert, in expert order.
+// pair_tok[q] is the token of pair q; pair_of[t*k + s] the pair of token t's
+// slot s; items the {expert, first pair, pairs, 0} of every tile of at most
+// `tile` pairs (all that the product kernels need to start on their loads).  The order of pairs within an expert does
 // not change any result: each pair's outputs depend only on its own row.
 constexpr int kBucketThreads = 1024;  // (the counting and scattering atomics spread wider)
 __global__ __launch_bounds__(kBucketThreads) void k_bucket(const int32_t* __restrict__ topk_idx, int m,
-                                                   int k, int n_expert, int* __restrict__ offsets,
-                                                   int* __restrict__ pair_tok,
+                                                   int k, int n_expert, int* __restrict__ pair_tok,
                                                    int* __restrict__ pair_of,
-                                                   int2* __restrict__ items,
+                                                   int4* __restrict__ items,
                                                    int* __restrict__ n_items, int tile) {
   __shared__ int cnt[256], cur[256];
   __shared__ int wsum[2][kBucketThreads / 64];
@@ -328,13 +327,9 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket(const int32_t* __rest
     ot += wsum[1][w];
   }
   if (t < n_expert) {
-    offsets[t] = oc;
     cur[t] = oc;
-    for (int i = 0; i < ct; ++i) items[ot + i] = make_int2(t, i * tile);
-    if (t == n_expert - 1) {
-      offsets[n_expert] = oc + c;
-      *n_items = ot + ct;
-    }
+    for (int i = 0; i < ct; ++i) items[ot + i] = make_int4(t, oc + i * tile, min(tile, c - i * tile), 0);
+    if (t == n_expert - 1) *n_items = ot + ct;
   }
   __syncthreads();
   for (int p = t; p < P; p += kBucketThreads) {
@@ -354,8 +349,7 @@ struct GroupArgs {
   const _Float16* sh;       // sub-block sums, high parts
   const _Float16* sl;
   int P;                    // pairs
-  const int* offsets;       // [E + 1]; null: dense, the P rows are one expert
-  const int2* items;
+  const int4* items;        // {expert, first pair, pairs, 0}; null: dense, the P rows are one expert
   const int* n_items;
   float* out;               // [pairs][n_out]
   const float* resid = nullptr;  // optional [pairs][n_out] added to out (may alias out)
@@ -366,9 +360,8 @@ struct GroupArgs {
   int ksplit = 1;
   float* partial = nullptr;
   int tile = kTok;          // pairs per work item of the list (<= kTok)
-  // gate/up of the few-pair kernel with 32 rows per workgroup: the output in
-  // k_split_tile's layout (f16 high parts, remainders, per-32 sums) instead
-  // of f32 rows, when oh is set
+  // gate/up: the output in k_split_tile's layout (f16 high parts, remainders,
+  // per-32 sums)
   _Float16 *oh = nullptr, *ol = nullptr, *osh = nullptr, *osl = nullptr;
 };
 
@@ -439,15 +432,15 @@ template <bool GATEUP, int NSBT = 0>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void k_group_q4k(GroupArgs a) {
   extern __shared__ uint4 lds[];
   // grouped: a work item of the list and a row block (xcd_item); dense (no
-  // offsets): the m rows are one expert, tile blockIdx.y, row block blockIdx.x
+  // items): the m rows are one expert, tile blockIdx.y, row block blockIdx.x
   int e = 0, p0 = blockIdx.y * kTok, cnt = min(kTok, a.P - p0), rblock = blockIdx.x;
-  if (a.offsets) {
+  if (a.items) {
     int item;
     if (!xcd_item(gridDim.x, *a.n_items, rblock, item)) return;  // uniform over the workgroup
-    const int2 it = a.items[item];
+    const int4 it = a.items[item];
     e = it.x;
-    p0 = a.offsets[e] + it.y;
-    cnt = min(a.tile, a.offsets[e + 1] - p0);
+    p0 = it.y;
+    cnt = it.z;
   }
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int rbase = rblock * kRowsWG + wave * 32;
@@ -719,6 +712,28 @@ __device__ __forceinline__ f32x4 mfma16(half8 a, half8 b, f32x4 c) {
 }
 
 
+// LDS DMA of 16 bytes per lane by asm, lane l's from g to LDS address
+// base + 16 l: the compiler's wait placement would make every LDS access after
+// a DMA that it knows of wait for it.  The kernel waits for its DMA itself
+// (vmcnt) before the barrier that hands the rows over; the compiler's own
+// counts only grow stricter by it.
+__device__ __forceinline__ uint32_t lds_addr(const void* p) {
+  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
+}
+__device__ __forceinline__ void dma16(const void* g, uint32_t base) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(g), "s"(base) : "memory");
+}
+constexpr int kLdsOnly = vm_lds_imm(63);
+// Workgroup barrier after the wait `imm` (__syncthreads() would wait for the
+// DMA in flight too).
+#define KNJ_FEW_BARRIER(imm)                \
+  do {                                      \
+    __builtin_amdgcn_s_waitcnt(imm);        \
+    __builtin_amdgcn_sched_barrier(0);      \
+    asm volatile("s_barrier" ::: "memory"); \
+    __builtin_amdgcn_sched_barrier(0);      \
+  } while (0)
+
 struct FewBlock {
   uint4 h, c0, c1;  // header (d, dmin, scales), the lane's 32 code bytes
 };
@@ -780,25 +795,22 @@ __device__ __forceinline__ void few_superblock(const FewBlock& b, const half8 (&
   for (int i = 0; i < 4; ++i) acc[i] += d * cq[i] - dmin * cm[i];
 }
 
-// The few-pair grouped product with the reduction split over the waves of a
-// workgroup: workgroup = (FT 16-row tiles of every matrix) x (up to 8 pairs of
+// The few-pair down product with the reduction split over the waves of a
+// workgroup: workgroup = (FT 16-row tiles) x (up to 8 pairs of
 // one expert); wave w takes super-blocks w, w + KS, ... (KS = waves, NSBW per
 // wave) and issues every load of them before any arithmetic, so a workgroup
 // asks for whole rows (all super-blocks) of its tiles at once.  The waves'
 // partial tiles meet in LDS and are added in wave order.
-template <bool GATEUP, int FT, int NSBW, bool SPLIT = false>
+template <int FT, int NSBW>
 __global__ __launch_bounds__(256) void k_group_fewk(GroupArgs a) {
-  static_assert(!SPLIT || (GATEUP && FT == 2), "split output: gate/up over 32 rows");
-  constexpr int NM = GATEUP ? 2 : 1;
-  __shared__ f32x4 part[4][NM * FT][64];
-  __shared__ float vs[SPLIT ? 32 : 1][kFew];  // the workgroup's outputs (split form)
+  __shared__ f32x4 part[4][FT][64];
   // (the plain order: the XCD-aware mapping of the 32-pair kernels measured
   // slower here, where an expert rarely has more than one item)
   const int item = blockIdx.y, rblock = blockIdx.x;
+  // (read with the count, not after it: the list holds gridDim.y entries)
+  const int4 it = a.items[item];
   if (item >= *a.n_items) return;  // uniform over the workgroup
-  const int2 it = a.items[item];
-  const int e = it.x, p0 = a.offsets[e] + it.y;
-  const int cnt = min(kFew, a.offsets[e + 1] - p0);
+  const int e = it.x, p0 = it.y, cnt = it.z;
   const int KS = blockDim.x >> 6;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int col = lane & 15, kq = lane >> 4;
@@ -813,7 +825,7 @@ __global__ __launch_bounds__(256) void k_group_fewk(GroupArgs a) {
   const _Float16* sbase = (apart ? a.sl : a.sh) + (uint64_t)ap * 8 + 2 * kq;
   const FewLane L(kq);
   struct Buf {
-    FewBlock w[NM][FT];
+    FewBlock w[FT];
     half8 x[8];
     uint32_t s2;
   };
@@ -823,16 +835,13 @@ __global__ __launch_bounds__(256) void k_group_fewk(GroupArgs a) {
     const int sb = wave + KS * i;
     if (sb < nsb) {  // uniform over the wave
 #pragma unroll
-      for (int mtx = 0; mtx < NM; ++mtx)
-#pragma unroll
-        for (int f = 0; f < FT; ++f) {
-          const int row = min(rbase + 16 * f + col, a.n_out - 1);
-          const uint8_t* p = (mtx ? a.w1 : a.w0) + (uint64_t)e * slab + (uint64_t)row * rb +
-                             (uint64_t)sb * KNJ_Q4K_BLOCK;
-          B[i].w[mtx][f].h = *reinterpret_cast<const uint4*>(p);
-          B[i].w[mtx][f].c0 = *reinterpret_cast<const uint4*>(p + KNJ_Q4K_QS + 32 * kq);
-          B[i].w[mtx][f].c1 = *reinterpret_cast<const uint4*>(p + KNJ_Q4K_QS + 32 * kq + 16);
-        }
+      for (int f = 0; f < FT; ++f) {
+        const int row = min(rbase + 16 * f + col, a.n_out - 1);
+        const uint8_t* p = a.w0 + (uint64_t)e * slab + (uint64_t)row * rb + (uint64_t)sb * KNJ_Q4K_BLOCK;
+        B[i].w[f].h = *reinterpret_cast<const uint4*>(p);
+        B[i].w[f].c0 = *reinterpret_cast<const uint4*>(p + KNJ_Q4K_QS + 32 * kq);
+        B[i].w[f].c1 = *reinterpret_cast<const uint4*>(p + KNJ_Q4K_QS + 32 * kq + 16);
+      }
 #pragma unroll
       for (int u = 0; u < 8; ++u)
         B[i].x[u] = ld_h8(abase + (uint64_t)(32 * sb + 8 * kq + 4 * (u & 1) + (u >> 1)) * P * 8);
@@ -840,11 +849,9 @@ __global__ __launch_bounds__(256) void k_group_fewk(GroupArgs a) {
     }
   }
   __builtin_amdgcn_sched_barrier(0);
-  f32x4 acc[NM][FT];
+  f32x4 acc[FT];
 #pragma unroll
-  for (int mtx = 0; mtx < NM; ++mtx)
-#pragma unroll
-    for (int f = 0; f < FT; ++f) acc[mtx][f] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int f = 0; f < FT; ++f) acc[f] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int i = 0; i < NSBW; ++i) {
     if (wave + KS * i < nsb) {
@@ -852,79 +859,190 @@ __global__ __launch_bounds__(256) void k_group_fewk(GroupArgs a) {
       xm[0] = as_h2(B[i].s2).x;
       xm[1] = as_h2(B[i].s2).y;
 #pragma unroll
-      for (int mtx = 0; mtx < NM; ++mtx)
-#pragma unroll
-        for (int f = 0; f < FT; ++f) few_superblock(B[i].w[mtx][f], B[i].x, xm, L, acc[mtx][f]);
+      for (int f = 0; f < FT; ++f) few_superblock(B[i].w[f], B[i].x, xm, L, acc[f]);
     }
   }
 #pragma unroll
-  for (int mtx = 0; mtx < NM; ++mtx)
-#pragma unroll
-    for (int f = 0; f < FT; ++f) part[wave][mtx * FT + f][lane] = acc[mtx][f];
+  for (int f = 0; f < FT; ++f) part[wave][f][lane] = acc[f];
   __syncthreads();
-  // wave w finishes tiles w, w + KS, ... of every matrix, the ranges added in
-  // wave order; lane's four values: pair 2 kq + i / 2, part i % 2, weight row
+  // wave w finishes tiles w, w + KS, ..., the ranges added in wave order; lane's four values: pair 2 kq + i / 2, part i % 2, weight row
   // 16 f + col
   for (int f = wave; f < FT; f += KS) {
     const int row = rbase + 16 * f + col;
     if (row >= a.n_out) continue;
-    f32x4 s[NM];
-#pragma unroll
-    for (int mtx = 0; mtx < NM; ++mtx) {
-      s[mtx] = part[0][mtx * FT + f][lane];
-      for (int w = 1; w < KS; ++w) s[mtx] += part[w][mtx * FT + f][lane];
-    }
+    f32x4 s = part[0][f][lane];
+    for (int w = 1; w < KS; ++w) s += part[w][f][lane];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int pj = 2 * kq + h;
-      if (pj >= cnt) continue;
-      float v = s[0][2 * h] + s[0][2 * h + 1];
-      if constexpr (GATEUP) {
-        const float u = s[NM - 1][2 * h] + s[NM - 1][2 * h + 1];
-        v = (v / (1.0f + expf(-v))) * u;
-      }
-      if (SPLIT) {
-        vs[16 * f + col][pj] = v;
-      } else {
-        const uint64_t o = (uint64_t)(p0 + pj) * a.n_out + row;
-        a.out[o] = a.resid ? a.resid[o] + v : v;
-      }
+      if (pj < cnt) a.out[(uint64_t)(p0 + pj) * a.n_out + row] = s[2 * h] + s[2 * h + 1];
     }
   }
-  if constexpr (SPLIT) {
-    // the 32 rows [rbase, rbase + 32) of every pair in k_split_tile's layout:
-    // thread (pair p, 8-group g) the group's high parts and remainders in
-    // perm8 order; the 32-row sum, split the same way, per pair
-    __syncthreads();
-    const int P = a.P, t = threadIdx.x;
-    if (t < 32) {
-      const int pp = t & 7, g = t >> 3;
-      if (pp < cnt) {
-        half8 h, l;
+}
+
+// The few-pair gate/up product with SwiGLU: workgroup = up to 8 pairs of one
+// expert x `units` units of 16 rows of both matrices, walked in order; wave w
+// takes super-blocks w, w + KS, ... (KS = waves, NSBW per wave), whose
+// activations stay in registers for all units.  A unit's rows reach LDS by DMA
+// while the unit before it is decoded from there (two buffers, two workgroups
+// of eight waves per CU).  The waves' partial tiles meet in LDS and are added
+// in wave order by one of them.  The output is in k_split_tile's layout.
+// Bound by the decoding's vector instructions (about 120 per 16-row tile and
+// super-block, 36 matrix-core cycles per four of them): 616 pairs over 128
+// experts of 768 x 2048 take 61.8 us (226 MB of weights, 3.7 TB/s).  One
+// workgroup per 32 rows with every load before any arithmetic, which could
+// overlap the two only across workgroups, took 69 us; this kernel with four
+// waves of two super-blocks each 63-65 us.
+//
+// A 16-row tile lies in LDS as groups of eight 16-byte pieces of every row (a
+// DMA instruction takes 128 contiguous bytes of eight rows); within its row's
+// 128 bytes a piece sits at its number xor row / 2, which spreads the 16 rows
+// that a read of one piece touches over all banks.
+template <int NSBW>
+__global__ __launch_bounds__(512, NSBW == 1 ? 4 : 2) void k_few_gateup(GroupArgs a, int units) {
+  extern __shared__ uint4 lds[];
+  // (the plain order: the XCD-aware mapping of the 32-pair kernels measured
+  // slower here, where an expert rarely has more than one item)
+  const int item = blockIdx.y;
+  // (read with the count, not after it: the list holds gridDim.y entries)
+  const int4 it = a.items[item];
+  if (item >= *a.n_items) return;  // uniform over the workgroup
+  const int e = it.x, p0 = it.y, cnt = it.z;
+  const int KS = blockDim.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, kq = lane >> 4;
+  const int nsb = a.n_in >> 8, np = 9 * nsb, ng = (np + 7) >> 3;  // 2 KB groups of a tile
+  const uint64_t P = (uint64_t)a.P;
+  const uint64_t rb = (uint64_t)nsb * KNJ_Q4K_BLOCK;
+  const uint64_t slab = rb * (uint64_t)a.n_out;
+  const int u0 = blockIdx.x * units, u1 = min(u0 + units, a.n_out / 16);
+  const uint32_t ubytes = (uint32_t)(2 * ng) << 11;
+  uint8_t* lb = reinterpret_cast<uint8_t*>(lds);
+  float2* part = reinterpret_cast<float2*>(lb + 2 * ubytes);  // [KS][2][64]
+  const uint32_t lds0 = lds_addr(lb);
+  // lane's row and piece of a DMA instruction
+  const int dr = lane >> 3, dq0 = (lane & 7) ^ (lane >> 4), dq1 = (lane & 7) ^ ((lane >> 4) + 4);
+  auto fetch = [&](int u, int buf) {
 #pragma unroll
-        for (int jj = 0; jj < 8; ++jj) {
-          const float x = vs[8 * g + perm8(jj)][pp];
-          h[jj] = (_Float16)x;
-          l[jj] = (_Float16)(x - (float)h[jj]);
+    for (int mf = 0; mf < 2; ++mf) {
+      const uint8_t* src = (mf ? a.w1 : a.w0) + (uint64_t)e * slab +
+                           (uint64_t)(16 * u + dr) * rb;
+      for (int g = wave; g < ng; g += KS) {
+        const uint32_t base = lds0 + buf * ubytes + ((uint32_t)(mf * ng + g) << 11);
+        dma16(src + 16 * min(8 * g + dq0, np - 1), __builtin_amdgcn_readfirstlane(base));
+        dma16(src + 8 * rb + 16 * min(8 * g + dq1, np - 1), __builtin_amdgcn_readfirstlane(base + 1024));
+      }
+    }
+  };
+  fetch(u0, 0);
+  // A row of this lane: pair ap (clamped into the item), part apart
+  const int ap = p0 + min(col >> 1, cnt - 1), apart = col & 1;
+  const _Float16* abase = (apart ? a.al : a.ah) + (uint64_t)ap * 8;
+  const _Float16* sbase = (apart ? a.sl : a.sh) + (uint64_t)ap * 8 + 2 * kq;
+  const FewLane L(kq);
+  half8 x[NSBW][8];
+  uint32_t s2[NSBW], oh[NSBW], o0[NSBW], o1[NSBW];
+#pragma unroll
+  for (int i = 0; i < NSBW; ++i) {
+    const int sb = min(wave + KS * i, nsb - 1);
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      x[i][u] = ld_h8(abase + (uint64_t)(32 * sb + 8 * kq + 4 * (u & 1) + (u >> 1)) * P * 8);
+    s2[i] = *reinterpret_cast<const uint32_t*>(sbase + (uint64_t)sb * P * 8);
+    auto at = [&](int pc) { return (uint32_t)((pc >> 3) << 11) + 128 * col + 16 * ((pc & 7) ^ (col >> 1)); };
+    oh[i] = at(9 * sb);
+    o0[i] = at(9 * sb + 1 + 2 * kq);
+    o1[i] = at(9 * sb + 2 + 2 * kq);
+  }
+  // A unit's results wait in its finishing wave's registers and are stored
+  // after the next barrier: a store right before it would have to complete
+  // there, where the wave waits for its part of the next unit's rows.
+  const int pp = lane & 7, pg = lane >> 3;  // pair and 8-group that the lane stores
+  half8 hv = {}, lv = {};
+  float sum32 = 0.0f;
+  int pend = -1;
+  auto store = [&](int u) {
+    if (pp < cnt && pg < 2) {
+      const uint64_t o = ((uint64_t)(2 * u + pg) * P + p0 + pp) * 8;
+      *reinterpret_cast<half8*>(a.oh + o) = hv;
+      *reinterpret_cast<half8*>(a.ol + o) = lv;
+    } else if (pp < cnt && pg == 4 && (u & 1)) {
+      const _Float16 sh = (_Float16)sum32;
+      const int b = u >> 1;
+      const uint64_t o = ((uint64_t)(b / 8) * P + p0 + pp) * 8 + b % 8;
+      a.osh[o] = sh;
+      a.osl[o] = (_Float16)(sum32 - (float)sh);
+    }
+  };
+  for (int u = u0; u < u1; ++u) {
+    const int buf = (u - u0) & 1;
+    // the unit's rows have landed, every wave is past the buffer that the
+    // next one fills
+    KNJ_FEW_BARRIER(vm_lds_imm(0));
+    if (u + 1 < u1) fetch(u + 1, buf ^ 1);
+    if (pend >= 0) store(pend);
+    pend = -1;
+    f32x4 acc[2];
+#pragma unroll
+    for (int mf = 0; mf < 2; ++mf) acc[mf] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < NSBW; ++i) {
+      if (wave + KS * i < nsb) {  // uniform over the wave
+        half8 xm = {};
+        xm[0] = as_h2(s2[i]).x;
+        xm[1] = as_h2(s2[i]).y;
+#pragma unroll
+        for (int mf = 0; mf < 2; ++mf) {
+          const uint8_t* t = lb + buf * ubytes + ((uint32_t)(mf * ng) << 11);
+          FewBlock w;
+          w.h = *reinterpret_cast<const uint4*>(t + oh[i]);
+          w.c0 = *reinterpret_cast<const uint4*>(t + o0[i]);
+          w.c1 = *reinterpret_cast<const uint4*>(t + o1[i]);
+          few_superblock(w, x[i], xm, L, acc[mf]);
         }
-        const uint64_t o = ((uint64_t)(rbase / 8 + g) * P + p0 + pp) * 8;
-        *reinterpret_cast<half8*>(a.oh + o) = h;
-        *reinterpret_cast<half8*>(a.ol + o) = l;
-      }
-    } else if (t < 40) {
-      const int pp = t - 32;
-      if (pp < cnt) {
-        float sum = 0.0f;
-#pragma unroll
-        for (int r = 0; r < 32; ++r) sum += vs[r][pp];
-        const _Float16 sh = (_Float16)sum;
-        const int b = rbase / 32;
-        const uint64_t o = ((uint64_t)(b / 8) * P + p0 + pp) * 8 + b % 8;
-        a.osh[o] = sh;
-        a.osl[o] = (_Float16)(sum - (float)sh);
       }
     }
+#pragma unroll
+    for (int mf = 0; mf < 2; ++mf)  // the products of the two parts of a pair's x together
+      part[(wave * 2 + mf) * 64 + lane] = make_float2(acc[mf][0] + acc[mf][1], acc[mf][2] + acc[mf][3]);
+    KNJ_FEW_BARRIER(kLdsOnly);
+    // one wave finishes the unit, the others go on to the next (the same wave
+    // for both units of 32 rows); lane's two values: pairs 2 kq and 2 kq + 1,
+    // weight row col
+    if (wave != (u >> 1) % KS) continue;
+    float2 g2 = part[lane], u2 = part[64 + lane];
+    for (int w = 1; w < KS; ++w) {
+      const float2 gw = part[(2 * w) * 64 + lane], uw = part[(2 * w + 1) * 64 + lane];
+      g2.x += gw.x;
+      g2.y += gw.y;
+      u2.x += uw.x;
+      u2.y += uw.y;
+    }
+    asm volatile("" ::: "memory");               // (part's space is reused)
+    float* vs = reinterpret_cast<float*>(part);  // [16][kFew]
+    vs[col * kFew + 2 * kq] = (g2.x / (1.0f + expf(-g2.x))) * u2.x;
+    vs[col * kFew + 2 * kq + 1] = (g2.y / (1.0f + expf(-g2.y))) * u2.y;
+    // the unit's 16 rows of every pair in k_split_tile's layout: lane (pair pp,
+    // 8-group pg) the group's high parts and remainders in perm8 order; per
+    // pair the sum of the 32 rows of two units, split the same way (one wave's
+    // LDS accesses are in order)
+    asm volatile("" ::: "memory");
+    if (pg < 2) {
+#pragma unroll
+      for (int jj = 0; jj < 8; ++jj) {
+        const float xv = vs[(8 * pg + perm8(jj)) * kFew + pp];
+        hv[jj] = (_Float16)xv;
+        lv[jj] = (_Float16)(xv - (float)hv[jj]);
+      }
+    } else if (pg == 4) {
+      if (!(u & 1)) sum32 = 0.0f;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) sum32 += vs[r * kFew + pp];
+    }
+    asm volatile("" ::: "memory");
+    pend = u;
   }
+  if (pend >= 0) store(pend);
 }
 
 // Q6_K down projection of the grouped MoE (d * sc * (q - 32) per weight,
@@ -936,7 +1054,7 @@ __global__ __launch_bounds__(256) void k_group_fewk(GroupArgs a) {
 // parts, remainders) start from zero and are added to the accumulator scaled
 // by d * sc_G.  Q6_K blocks are 210 bytes, so the lane's byte runs are read
 // as aligned words and shifted into place (ld8_u2).  ksplit 1, no residual.
-// With null offsets the P rows are one expert (a dense product, e.g. a Q6_K
+// With null items the P rows are one expert (a dense product, e.g. a Q6_K
 // LM head over a batch of rows).
 struct Q6WBlock {
   uint32_t la[2][2][2], lb[2][2][2], qh[2][2][2];  // [half n][16-run lh][word]: ql +0, ql +32, qh
@@ -946,16 +1064,16 @@ struct Q6WBlock {
 
 __global__ __launch_bounds__(kBlock) void k_group_q6k(GroupArgs a) {
   extern __shared__ uint4 lds[];
-  // grouped: work item blockIdx.y; dense (no offsets): tile blockIdx.y of the
+  // grouped: work item blockIdx.y; dense (no items): tile blockIdx.y of the
   // P rows seen as one expert
   int e = 0, p0 = blockIdx.y * kTok, cnt = min(kTok, a.P - p0), rblock = blockIdx.x;
-  if (a.offsets) {
+  if (a.items) {
     int item;
     if (!xcd_item(gridDim.x, *a.n_items, rblock, item)) return;  // uniform over the workgroup
-    const int2 it = a.items[item];
+    const int4 it = a.items[item];
     e = it.x;
-    p0 = a.offsets[e] + it.y;
-    cnt = min(a.tile, a.offsets[e + 1] - p0);
+    p0 = it.y;
+    cnt = it.z;
   }
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int rbase = rblock * kRowsWG + wave * 32;
@@ -1442,9 +1560,8 @@ uint64_t moe_batch_scratch_bytes(int m, int n_embd, int n_ff, int n_expert, int 
   add(m * H * 4);                       // hx
   add(P * H * 2); add(P * H * 2);       // x hi/lo per pair
   add(P * H / 16); add(P * H / 16);     // x sums hi/lo
-  add((n_expert + 1) * 4);              // offsets
   add(P * 4); add(P * 4);               // pair_tok, pair_of
-  add(items * 8); add(256);             // items, n_items
+  add(items * 16); add(256);            // items, n_items
   add(P * F * 4);                       // act
   add(P * F * 2); add(P * F * 2);       // act hi/lo
   add(P * F / 16); add(P * F / 16);     // act sums hi/lo
@@ -1473,26 +1590,45 @@ hipError_t group_lds_attr() {
   return e;
 }
 
-// The few-pair product over n_in: KS = min(4, super-blocks) waves per
-// workgroup, each with NSBW super-blocks; ft 16-row tiles per workgroup.
-template <bool GATEUP>
-hipError_t launch_fewk(const GroupArgs& g, int max_items, int ft, hipStream_t s) {
-  const int nsb = g.n_in >> 8, ks = std::min(4, nsb), nw = (nsb + ks - 1) / ks;
-  const dim3 grid((g.n_out + 16 * ft - 1) / (16 * ft), max_items), block(64 * ks);
-#define KNJ_FEWK(FT, NW) \
-  if (ft == FT && nw <= NW) { KNJ_LAUNCH((k_group_fewk<GATEUP, FT, NW>), grid, block, 0, s, g); return hipGetLastError(); }
-  if constexpr (GATEUP) {
-    if (g.oh) {  // the split output (32 rows per workgroup)
-      if (ft != 2 || g.n_out % 32) return hipErrorInvalidValue;
-      if (nw <= 1) { KNJ_LAUNCH((k_group_fewk<GATEUP, 2, 1, true>), grid, block, 0, s, g); return hipGetLastError(); }
-      if (nw <= 2) { KNJ_LAUNCH((k_group_fewk<GATEUP, 2, 2, true>), grid, block, 0, s, g); return hipGetLastError(); }
-      if (nw <= 4) { KNJ_LAUNCH((k_group_fewk<GATEUP, 2, 4, true>), grid, block, 0, s, g); return hipGetLastError(); }
-      return hipErrorInvalidValue;
-    }
-  }
-  KNJ_FEWK(2, 1) KNJ_FEWK(2, 2) KNJ_FEWK(2, 4) KNJ_FEWK(4, 1)
-#undef KNJ_FEWK
-  return hipErrorInvalidValue;
+// The few-pair gate/up product: KS = min(8, super-blocks) waves per workgroup.
+template <int NSBW>
+hipError_t launch_few_gateup_as(const GroupArgs& g, int max_items, hipStream_t s) {
+  static const hipError_t attr =
+      hipFuncSetAttribute((const void*)k_few_gateup<NSBW>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 << 10);
+  if (attr != hipSuccess) return attr;
+  const int nsb = g.n_in >> 8, ks = std::min(8, nsb), ng = (9 * nsb + 7) / 8;
+  const size_t lds = (size_t)(8 * ng + ks) << 10;  // two buffers of two tiles, the partial sums
+  // units per workgroup, an even number: more of them share the wait for the
+  // first, fewer fill the last round of workgroups (77 tokens / 32 sequences
+  // of the 768 x 2048 experts, whole layer and step: 117.9 us / 751 us with 4,
+  // 117.4 / 745 with 6, 119.8 / 745 with 8, 126.9 / 735 with 12, 120.2 / 785
+  // with 16)
+  const int units = 6;
+  KNJ_LAUNCH(k_few_gateup<NSBW>, dim3((g.n_out / 16 + units - 1) / units, max_items), dim3(64 * ks), lds, s, g,
+             units);
+  return hipGetLastError();
+}
+hipError_t launch_few_gateup(const GroupArgs& g, int max_items, hipStream_t s) {
+  if (g.n_in % 256 || g.n_in <= 0 || g.n_in > 4096 || g.n_out % 32 || !g.oh) return hipErrorInvalidValue;
+  return g.n_in <= 8 * 256 ? launch_few_gateup_as<1>(g, max_items, s) : launch_few_gateup_as<2>(g, max_items, s);
+}
+
+// The few-pair down product: KS = min(4, super-blocks) waves per workgroup,
+// each with NSBW super-blocks of FT 16-row tiles.
+template <int FT, int NSBW>
+hipError_t launch_fewk_as(const GroupArgs& g, int max_items, hipStream_t s) {
+  KNJ_LAUNCH((k_group_fewk<FT, NSBW>), dim3((g.n_out + 16 * FT - 1) / (16 * FT), max_items),
+             dim3(64 * std::min(4, g.n_in >> 8)), 0, s, g);
+  return hipGetLastError();
+}
+hipError_t launch_fewk(const GroupArgs& g, int max_items, hipStream_t s) {
+  const int nsb = g.n_in >> 8;
+  if (nsb <= 0 || nsb > 16) return hipErrorInvalidValue;
+  // (measured at 32 sequences with one super-block per wave: 64 rows per
+  // workgroup)
+  if (nsb <= 4) return launch_fewk_as<4, 1>(g, max_items, s);
+  if (nsb <= 8) return launch_fewk_as<2, 2>(g, max_items, s);
+  return launch_fewk_as<2, 4>(g, max_items, s);
 }
 
 hipError_t launch_moe_batch(const MoeBatchArgs& a, void* scratch, hipStream_t s) {
@@ -1518,10 +1654,9 @@ hipError_t launch_moe_batch(const MoeBatchArgs& a, void* scratch, hipStream_t s)
   _Float16* xl = (_Float16*)take(P * H * 2);
   _Float16* sxh = (_Float16*)take(P * H / 16);
   _Float16* sxl = (_Float16*)take(P * H / 16);
-  int* offsets = (int*)take((uint64_t)(E + 1) * 4);
   int* pair_tok = (int*)take(P * 4);
   int* pair_of = (int*)take(P * 4);
-  int2* items = (int2*)take((uint64_t)max_items * 8);
+  int4* items = (int4*)take((uint64_t)max_items * 16);
   int* n_items = (int*)take(256);
   float* act = (float*)take(P * F * 4);
   _Float16* ah = (_Float16*)take(P * F * 2);
@@ -1541,21 +1676,19 @@ hipError_t launch_moe_batch(const MoeBatchArgs& a, void* scratch, hipStream_t s)
              s, xin, a.router_w, m, H, E, rpart);
   KNJ_LAUNCH(k_route_batch, dim3((m + 3) / 4), dim3(kBlock), 0, s, rpart, kz, m, E, K, a.logits,
              a.topk_idx, a.topk_w);
-  KNJ_LAUNCH(k_bucket, dim3(1), dim3(kBucketThreads), 0, s, a.topk_idx, m, K, E, offsets, pair_tok,
+  KNJ_LAUNCH(k_bucket, dim3(1), dim3(kBucketThreads), 0, s, a.topk_idx, m, K, E, pair_tok,
                      pair_of, items, n_items, tile);
   KNJ_LAUNCH(k_split_tile, dim3((unsigned)((P + 31) / 32), H / 64), dim3(kBlock), 0, s, xin,
              pair_tok, H, (int)P, xh, xl, sxh, sxl);
-  GroupArgs gu{a.gate, a.up, H, F, xh, xl, sxh, sxl, (int)P, offsets, items, n_items, act};
+  GroupArgs gu{a.gate, a.up, H, F, xh, xl, sxh, sxl, (int)P, items, n_items, act};
   gu.tile = tile;
-  // (measured at 32 sequences: 32 rows per workgroup for gate/up, whose
-  // super-blocks fill two per wave; 64 for down, one per wave)
   if (few) {
     // SwiGLU written straight in the down product's operand layout
     gu.oh = ah;
     gu.ol = al;
     gu.osh = sah;
     gu.osl = sal;
-    if (hipError_t e = launch_fewk<true>(gu, max_items, 2, s)) return e;
+    if (hipError_t e = launch_few_gateup(gu, max_items, s)) return e;
   } else {
     // SwiGLU written straight in the down product's operand layout
     gu.oh = ah;
@@ -1565,10 +1698,10 @@ hipError_t launch_moe_batch(const MoeBatchArgs& a, void* scratch, hipStream_t s)
     KNJ_LAUNCH(k_group_q4k<true>, dim3((F + kRowsWG - 1) / kRowsWG, max_items + 8), dim3(kBlock),
                kGroupLds, s, gu);
   }
-  GroupArgs dn{a.down, nullptr, F, H, ah, al, sah, sal, (int)P, offsets, items, n_items, y};
+  GroupArgs dn{a.down, nullptr, F, H, ah, al, sah, sal, (int)P, items, n_items, y};
   dn.tile = tile;
   if (few && a.type_down == KNJ_TYPE_Q4_K) {
-    if (hipError_t e = launch_fewk<false>(dn, max_items, (F >> 8) <= 4 ? 4 : 2, s)) return e;
+    if (hipError_t e = launch_fewk(dn, max_items, s)) return e;
   } else if (a.type_down == KNJ_TYPE_Q6_K)
     KNJ_LAUNCH(k_group_q6k, dim3((H + kRowsWG - 1) / kRowsWG, max_items + 8), dim3(kBlock), kGroupLds,
                s, dn);
@@ -1667,7 +1800,7 @@ hipError_t launch_dense_q4k_ex(const uint8_t* w, int n_in, int n_out, int m, con
                n_in, m, const_cast<_Float16*>(xh), const_cast<_Float16*>(xl),
                const_cast<_Float16*>(sh), const_cast<_Float16*>(sl));
   }
-  GroupArgs g{w, nullptr, n_in, n_out, xh, xl, sh, sl, m, nullptr, nullptr, nullptr, out, resid};
+  GroupArgs g{w, nullptr, n_in, n_out, xh, xl, sh, sl, m, nullptr, nullptr, out, resid};
   g.ksplit = ks;
   g.partial = part;
   const int tiles = (m + kTok - 1) / kTok;
@@ -1723,7 +1856,7 @@ hipError_t launch_dense_q6k(const uint8_t* w, int n_in, int n_out, int m, const 
   _Float16* sl = (_Float16*)take(P * n_in / 16);
   KNJ_LAUNCH(k_split_tile, dim3((m + 31) / 32, n_in / 64), dim3(kBlock), 0, s, x, nullptr,
              n_in, m, xh, xl, sh, sl);
-  GroupArgs g{w, nullptr, n_in, n_out, xh, xl, sh, sl, m, nullptr, nullptr, nullptr, out, nullptr};
+  GroupArgs g{w, nullptr, n_in, n_out, xh, xl, sh, sl, m, nullptr, nullptr, out, nullptr};
   KNJ_LAUNCH(k_group_q6k, dim3((n_out + kRowsWG - 1) / kRowsWG, (m + kTok - 1) / kTok),
              dim3(kBlock), kGroupLds, s, g);
   return hipGetLastError();

@@ -73,3 +73,32 @@ def test_batch_bf16_head_edges(device, n_embd, n_vocab, B):
     batch.close()
     assert np.array_equal(np.asarray(first).reshape(-1), lg.argmax(axis=1))
     gm.close()
+
+
+@pytest.mark.parametrize("n_embd,n_ff,m", [(256, 256, 1), (768, 512, 9), (2304, 768, 5), (4096, 256, 12), (1024, 1280, 3)])
+def test_moe_few_pairs_edges(device, n_embd, n_ff, m):
+    """The few-pair expert products (fewer than ten pairs per expert) at one
+    super-block, at counts of super-blocks that the waves of a workgroup share
+    unevenly, at the widest row, at row counts that leave the last workgroup a
+    remainder, and with items of one to eight pairs and more than one item per
+    expert: against the oracle within the parity bar (1e-5)."""
+    n_expert, k = 8, 4
+    print(f"few pairs {n_embd}x{n_ff} m={m}", flush=True)
+    syn = lambda kind, t, a, b, e=-1: O.synth_tensor(O.tensor_key(SEED, 1, kind, e), t, a, b)
+    router = syn("router", K.TYPE_F32, n_embd, n_expert)
+    gate, up = (np.concatenate([syn(n, K.TYPE_Q4_K, n_embd, n_ff, e) for e in range(n_expert)]) for n in ("gate", "up"))
+    down = np.concatenate([syn("down", K.TYPE_Q4_K, n_ff, n_embd, e) for e in range(n_expert)])
+    rng = np.random.default_rng(n_embd + m)
+    # (tokens 8 and later repeat the first: nine pairs and more on its experts)
+    x = rng.standard_normal((m, n_embd)).astype(np.float32)
+    x[8:] = x[0]
+    resid = rng.standard_normal((m, n_embd)).astype(np.float32)
+    want, _, ti_w, _ = O.moe(x, router, gate, up, down, n_embd, n_ff, n_expert, k, type_down=K.TYPE_Q4_K)
+    d = [K.DeviceBuffer.from_array(a) for a in (x, router, gate, up, down)]
+    out, logits = K.DeviceBuffer(4 * m * n_embd), K.DeviceBuffer(4 * m * n_expert)
+    ti, tw = K.DeviceBuffer(4 * m * k), K.DeviceBuffer(4 * m * k)
+    K.moe_batch_layer(*d, m, n_embd, n_ff, n_expert, k, out, logits, ti, tw, resid=K.DeviceBuffer.from_array(resid))
+    assert np.array_equal(ti.download(np.int32).reshape(m, k), ti_w)
+    got = out.download(np.float32).reshape(m, n_embd) - resid
+    for t in range(m):
+        assert rel_rmse(got[t], want[t]) <= 1e-5, t
