@@ -1052,17 +1052,25 @@ __global__ __launch_bounds__(512, NSBW == 1 ? 4 : 2) void k_few_gateup(GroupArgs
 // of its row (in the staging's perm8 order) as exact f16 values q - 32, and
 // reads the activations of 8-group 2 G + kh.  A step's two products (high
 // parts, remainders) start from zero and are added to the accumulator scaled
-// by d * sc_G.  Q6_K blocks are 210 bytes, so the lane's byte runs are read
-// as aligned words and shifted into place (ld8_u2).  ksplit 1, no residual.
+// by d * sc_G.  Q6_K blocks are 210 bytes: the lane's code
+// bytes come in 16-byte pieces at 2-byte aligned addresses.  ksplit 1, no
+// residual.
+// Bound by the matrix cores and the vector instructions together: per step
+// 64 matrix-core cycles and 16 scaled additions, 17 decoding and 3 scale
+// instructions.  8000 pairs over 128 experts of 2048 x 768: 215 us with the
+// products in accumulation registers (16 reads a step, hence
+// amdgpu_waves_per_eu), masks as literals, 8-byte loads and a wait for the
+// next block's DMA before this block's reads; 197-206 us now, a 1500-token
+// chunk's 135 -> 120 us.
 // With null items the P rows are one expert (a dense product, e.g. a Q6_K
 // LM head over a batch of rows).
 struct Q6WBlock {
-  uint32_t la[2][2][2], lb[2][2][2], qh[2][2][2];  // [half n][16-run lh][word]: ql +0, ql +32, qh
+  uint32_t la[2][4], lb[2][4], qh[2][4];  // [16-run lh][2 half n + word]: ql +0, ql +32, qh
   uint32_t sc[4];                                   // the 16 int8 scales
   uint32_t d;                                       // f16 bits
 };
 
-__global__ __launch_bounds__(kBlock) void k_group_q6k(GroupArgs a) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2, 4))) void k_group_q6k(GroupArgs a) {
   extern __shared__ uint4 lds[];
   // grouped: work item blockIdx.y; dense (no items): tile blockIdx.y of the
   // P rows seen as one expert
@@ -1075,7 +1083,7 @@ __global__ __launch_bounds__(kBlock) void k_group_q6k(GroupArgs a) {
     p0 = it.y;
     cnt = it.z;
   }
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int rbase = rblock * kRowsWG + wave * 32;
   const bool rows_ok = rbase < a.n_out;
   const int row = min(rbase + (lane & 31), a.n_out - 1), kh = lane >> 5;
@@ -1091,23 +1099,33 @@ __global__ __launch_bounds__(kBlock) void k_group_q6k(GroupArgs a) {
       const int e0 = (8 * wave + u) * 64, ee = e0 + lane;
       const int part = ee >> 10, r = ee & 1023, q = r >> 5, jj = r & 31;
       const _Float16* src = (part ? a.al : a.ah) + ((uint64_t)(32 * sb + q) * P + p0 + min(jj, cnt - 1)) * 8;
-      __builtin_amdgcn_global_load_lds((glb_void*)src, (lds_void*)(lds + buf * kBuf + e0), 16, 0, 0);
+      dma16(src, __builtin_amdgcn_readfirstlane(lds_addr(lds + buf * kBuf + e0)));
     }
   };
+  // lane half kh loads the code bytes of the block's half kh, in 16-byte
+  // pieces; `spread` then hands each lane half its 8 bytes of both
   auto w_load = [&](int sb, Q6WBlock& w) {
     const uint8_t* b = wr + (uint64_t)sb * KNJ_Q6K_BLOCK;
 #pragma unroll
-    for (int n = 0; n < 2; ++n)
-#pragma unroll
-      for (int lh = 0; lh < 2; ++lh) {
-        const int l = 16 * lh + 8 * kh;
-        ld8_u2(b + KNJ_Q6K_QL + 64 * n + l, w.la[n][lh][0], w.la[n][lh][1]);
-        ld8_u2(b + KNJ_Q6K_QL + 64 * n + 32 + l, w.lb[n][lh][0], w.lb[n][lh][1]);
-        ld8_u2(b + KNJ_Q6K_QH + 32 * n + l, w.qh[n][lh][0], w.qh[n][lh][1]);
-      }
-    ld8_u2(b + KNJ_Q6K_SC, w.sc[0], w.sc[1]);
-    ld8_u2(b + KNJ_Q6K_SC + 8, w.sc[2], w.sc[3]);
+    for (int lh = 0; lh < 2; ++lh) {
+      __builtin_memcpy(w.la[lh], b + KNJ_Q6K_QL + 64 * kh + 16 * lh, 16);
+      __builtin_memcpy(w.lb[lh], b + KNJ_Q6K_QL + 64 * kh + 32 + 16 * lh, 16);
+      __builtin_memcpy(w.qh[lh], b + KNJ_Q6K_QH + 32 * kh + 16 * lh, 16);
+    }
+    __builtin_memcpy(w.sc, b + KNJ_Q6K_SC, 16);
     w.d = *reinterpret_cast<const uint16_t*>(b + KNJ_Q6K_D);
+  };
+  auto spread = [&](uint32_t (&r)[2][4]) {
+#pragma unroll
+    for (int lh = 0; lh < 2; ++lh)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        // words i and 2 + i: bytes 0-7 and 8-15 of half kh -> this lane
+        // half's bytes of half 0 and of half 1
+        const auto p = __builtin_amdgcn_permlane32_swap(r[lh][i], r[lh][2 + i], false, false);
+        r[lh][i] = p[0];
+        r[lh][2 + i] = p[1];
+      }
   };
   Q6WBlock wc, wn;
   stage(0, 0);
@@ -1116,7 +1134,12 @@ __global__ __launch_bounds__(kBlock) void k_group_q6k(GroupArgs a) {
   __syncthreads();
   f32x16 acc = {};
   const half2v bias = half2v{(_Float16)1056.0f, (_Float16)1056.0f};  // 1024 + 32
-  auto cv = [&](uint32_t w) { return as_h2((w & 0x00FF00FFu) | 0x64006400u) - bias; };
+  // masks and f16 exponent in registers: (x & mask) | y is one instruction then
+  uint32_t mb = 0x00FF00FFu, base = 0x64006400u, ml = 0x0F0F0F0Fu, mh = 0x30303030u;
+  asm volatile("" : "+v"(mb), "+v"(base), "+v"(ml), "+v"(mh));
+  auto cv = [&](uint32_t w) { return as_h2((w & mb) | base) - bias; };
+  // the two high code bits of quarter s4 at bits 4, 5 of every byte
+  auto hi = [&](uint32_t w, int s4) { return (s4 == 0 ? w << 4 : s4 == 1 ? w << 2 : s4 == 2 ? w : w >> 2) & mh; };
   for (int sb = 0; sb < nsb; ++sb) {
     const int buf = sb & 1;
     const int nx = min(sb + 1, nsb - 1);  // the last iteration reloads its own block, unused
@@ -1126,6 +1149,9 @@ __global__ __launch_bounds__(kBlock) void k_group_q6k(GroupArgs a) {
     __builtin_amdgcn_sched_barrier(0);
     const uint4* L = lds + buf * kBuf;
     const float d = h2f(wc.d);
+    spread(wc.la);
+    spread(wc.lb);
+    spread(wc.qh);
 #pragma unroll
     for (int n = 0; n < 2; ++n)
 #pragma unroll
@@ -1133,10 +1159,10 @@ __global__ __launch_bounds__(kBlock) void k_group_q6k(GroupArgs a) {
 #pragma unroll
         for (int s4 = 0; s4 < 4; ++s4) {
           const int G = 8 * n + 2 * s4 + lh;  // weights 16 G .. 16 G + 15
-          const uint32_t* ql = (s4 & 1) ? wc.lb[n][lh] : wc.la[n][lh];
-          const int nsh = 4 * (s4 >> 1), hsh = 2 * s4;
-          const uint32_t q0 = ((ql[0] >> nsh) & 0x0F0F0F0Fu) | (((wc.qh[n][lh][0] >> hsh) & 0x03030303u) << 4);
-          const uint32_t q1 = ((ql[1] >> nsh) & 0x0F0F0F0Fu) | (((wc.qh[n][lh][1] >> hsh) & 0x03030303u) << 4);
+          const uint32_t* ql = ((s4 & 1) ? wc.lb[lh] : wc.la[lh]) + 2 * n;
+          const int nsh = 4 * (s4 >> 1);
+          const uint32_t q0 = ((ql[0] >> nsh) & ml) | hi(wc.qh[lh][2 * n], s4);
+          const uint32_t q1 = ((ql[1] >> nsh) & ml) | hi(wc.qh[lh][2 * n + 1], s4);
           const half2v b0 = cv(q0), b1 = cv(q0 >> 8), b2 = cv(q1), b3 = cv(q1 >> 8);
           const half8 bw = half8{b0.x, b0.y, b1.x, b1.y, b2.x, b2.y, b3.x, b3.y};
           const half8 xh = __builtin_bit_cast(half8, L[(2 * G + kh) * kQStride + j]);
