@@ -207,55 +207,56 @@ __global__ __launch_bounds__(kBlock) void k_gemv_q4k_wide(const uint8_t* __restr
 
 // Q6_K rows of n_in <= 4096: LPR lanes per row, each with 64 weights of one
 // super-block: half hf, 16-run o of its four quarters (weights 128 hf + 32 t +
-// 16 o + i, t < 4, i < 16), which share one scale per quarter.  The lane's x
-// (64 values and 4 run sums) is the same for every row and stays in registers;
-// rows walked grid-stride (the argmax variant keeps the grid <= kMaxKeys).
+// 16 o + i, t < 4, i < 16), which share one scale per quarter.  The lane's 64 x
+// are the same for every row and stay in registers; rows walked grid-stride
+// (the argmax variant keeps the grid <= kMaxKeys).
+// The codes become signed values before any product: sums of q x with 32 sum x
+// taken off at the end carry the rounding of the larger terms (against float64
+// 2.2e-7 instead of 1.1e-7 at 2048 and 4096 inputs, 1.6e-7 instead of 0.8e-7
+// at 2304).
 // A lane reads its codes as three 16-byte pieces at 2-byte aligned addresses.
 // Bound by the vector memory unit and the vector instructions together.  With
 // 32 weights per lane, in 8-byte pieces (each as three aligned words), a row
-// took 14 loads of about 20 vector cache accesses and 4.9 vector instructions
-// a weight; now 5 loads serve two rows and 3.1 instructions a weight: the
-// 151,936 x 2048 head 60.5 -> 47.5 us (4.2 -> 5.4 TB/s).  Also measured there:
-// two and four rows per lane in flight 50.0 and 55.0 us, rows fetched into LDS
-// by DMA and decoded from there 76 us.
+// took 14 loads of about 20 vector cache accesses; now 5 loads serve two rows
+// and 234 vector instructions a lane's 64 weights: the 151,936 x 2048 head
+// 60.5 -> 48.6 us (4.2 -> 5.3 TB/s).  (Unsigned codes convert by shorter
+// instructions: 47.5 us, but see above.)  Also measured there with those: two
+// and four rows per lane in flight 50.0 and 55.0 us, rows fetched into LDS by
+// DMA and decoded from there 76 us.
 struct Q6Run {
   uint4 l0, l1, h;   // ql bytes of quarters 0 and 2, of 1 and 3, qh bytes
   uint32_t sa, sb;   // the half's 8 scales; quarter t's is byte 2 t + o
   uint32_t d;        // f16 bits of d
 };
 
-__device__ __forceinline__ Q6Run q6_run_load(const uint8_t* __restrict__ blk, int hf, int o) {
-  Q6Run r;
-  __builtin_memcpy(&r.l0, blk + KNJ_Q6K_QL + 64 * hf + 16 * o, 16);
-  __builtin_memcpy(&r.l1, blk + KNJ_Q6K_QL + 64 * hf + 32 + 16 * o, 16);
-  __builtin_memcpy(&r.h, blk + KNJ_Q6K_QH + 32 * hf + 16 * o, 16);
-  ld8_u2(blk + KNJ_Q6K_SC + 8 * hf, r.sa, r.sb);
-  r.d = *reinterpret_cast<const uint16_t*>(blk + KNJ_Q6K_D);
-  return r;
-}
-
-// sum over the run's 64 weights of w*x = d * sum_t sc_t * (sum_i q x - 32 sum_i x)
-__device__ __forceinline__ float q6_run_dot(const Q6Run& r, int o, const float (&x)[4][16], const float (&sx)[4]) {
+// sum over the run's 64 weights of w*x = d * sum_t sc_t * sum_i (q - 32) x
+__device__ __forceinline__ float q6_run_dot(const Q6Run& r, int o, const float (&x)[4][16]) {
   const uint32_t sh = 8 * o;
+  const uint32_t hw[4] = {r.h.x, r.h.y, r.h.z, r.h.w};
+  // (constants in registers: with literals the three-input operations split)
+  uint32_t ml = 0x3C3C3C3Cu, mq = 0xFCFCFCFCu, top = 0x80808080u;
+  asm("" : "+s"(ml), "+s"(mq), "+v"(top));
   float sum = 0.0f;
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
     const uint4 l = (t & 1) ? r.l1 : r.l0;
-    const uint32_t lw[4] = {l.x, l.y, l.z, l.w}, hw[4] = {r.h.x, r.h.y, r.h.z, r.h.w};
-    float a4[4] = {};  // (short chains: four of four terms)
+    const uint32_t lw[4] = {l.x, l.y, l.z, l.w};
+    float a[2] = {};  // (short chains: two of eight terms)
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      const uint32_t q = ((lw[k] >> (4 * (t >> 1))) & 0x0F0F0F0Fu) | (((hw[k] >> (2 * t)) & 0x03030303u) << 4);
-      a4[k] += (float)(q & 0xFFu) * x[t][4 * k];
-      a4[k] += (float)((q >> 8) & 0xFFu) * x[t][4 * k + 1];
-      a4[k] += (float)((q >> 16) & 0xFFu) * x[t][4 * k + 2];
-      a4[k] += (float)(q >> 24) * x[t][4 * k + 3];
+      // a code at bits 7 .. 2 of its byte with its top bit flipped: 4 (q - 32)
+      // as a signed byte
+      const uint32_t lo = (t & 2) ? lw[k] >> 2 : lw[k] << 2, hi = hw[k] << (6 - 2 * t);
+      const uint32_t q = (((lo & ml) | (hi & ~ml)) & mq) ^ top;
+      a[k & 1] += (float)(int8_t)q * x[t][4 * k];
+      a[k & 1] += (float)(int8_t)(q >> 8) * x[t][4 * k + 1];
+      a[k & 1] += (float)(int8_t)(q >> 16) * x[t][4 * k + 2];
+      a[k & 1] += (float)(int8_t)(q >> 24) * x[t][4 * k + 3];
     }
-    const float acc = (a4[0] + a4[1]) + (a4[2] + a4[3]);
     const float sc = (float)(int8_t)(((t & 2) ? r.sb : r.sa) >> (16 * (t & 1) + sh));
-    sum += sc * (acc - 32.0f * sx[t]);
+    sum += sc * (a[0] + a[1]);
   }
-  return h2f(r.d) * sum;
+  return 0.25f * h2f(r.d) * sum;  // (the quarter is exact: d is an f16)
 }
 
 template <int LPR>
@@ -265,49 +266,54 @@ __global__ __launch_bounds__(kBlock, 4) void k_gemv_q6k_u(const uint8_t* __restr
                                                        const float* __restrict__ resid,
                                                        float* __restrict__ y,
                                                        unsigned long long* argmax) {
-  __shared__ float xs[xpad_size(4096)];
-  __shared__ float xs16[256];
+  __shared__ float4 xs4[xpad_size(4096) / 4];
   __shared__ float red[8];
   constexpr int RPW = 64 / LPR;  // rows of a row-step
-  stage_x(x, nw, eps, n_in, xs, red);
-  for (int g = threadIdx.x; 16 * g < n_in; g += kBlock) {
-    float s = 0.0f;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const float4 a = *reinterpret_cast<const float4*>(xs + xpad(16 * g) + 4 * k);
-      s += (a.x + a.y) + (a.z + a.w);
-    }
-    xs16[g] = s;
-  }
-  __syncthreads();
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  stage_x(x, nw, eps, n_in, reinterpret_cast<float*>(xs4), red);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int sub = lane % LPR, rsub = lane / LPR;
   const int nb = n_in / KNJ_QK;
   const bool active = sub < 4 * nb;
   const int u = active ? sub : 0, b = u >> 2, hf = (u >> 1) & 1, o = u & 1;
-  float xv[4][16], sx[4];
+  float xv[4][16];
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
     const int i = 256 * b + 128 * hf + 32 * t + 16 * o;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      const float4 a = *reinterpret_cast<const float4*>(xs + xpad(i) + 4 * k);
+      const float4 a = xs4[xpad(i) / 4 + k];  // (whole 16-byte reads: the pad keeps those off one bank)
       xv[t][4 * k] = a.x;
       xv[t][4 * k + 1] = a.y;
       xv[t][4 * k + 2] = a.z;
       xv[t][4 * k + 3] = a.w;
     }
-    sx[t] = xs16[i >> 4];
   }
   const uint64_t rb = (uint64_t)nb * KNJ_Q6K_BLOCK;
-  const uint8_t* wu = w + (uint64_t)b * KNJ_Q6K_BLOCK;
+  // the lane's bytes from the step's first row, which is the wave's
+  uint32_t ob = rsub * (uint32_t)rb + b * KNJ_Q6K_BLOCK;
+  uint32_t ol = ob + KNJ_Q6K_QL + 64 * hf + 16 * o, oh = ob + KNJ_Q6K_QH + 32 * hf + 16 * o;
+  uint32_t os = ob + KNJ_Q6K_SC + 8 * hf;
   unsigned long long best = 0;
   const int stride = gridDim.x * (kBlock / 64) * RPW;
   for (int r0 = (blockIdx.x * (kBlock / 64) + wave) * RPW; r0 < n_out; r0 += stride) {
-    const int row = r0 + rsub, rc = min(row, n_out - 1);
-    const Q6Run q = q6_run_load(wu + (uint64_t)rc * rb, hf, o);
-    const float rv = resid ? resid[rc] : 0.0f;
-    const float acc = group_sum<LPR>(active ? q6_run_dot(q, o, xv, sx) : 0.0f);
+    const int row = r0 + rsub;
+    const uint8_t* wr = w + (uint64_t)r0 * rb;
+    float acc = 0.0f, rv = 0.0f;
+    if (active && row < n_out) {
+      // (32-bit offsets from a scalar base, kept so: hoisted, their extensions
+      // would make every address a 64-bit addition)
+      asm("" : "+v"(ob), "+v"(ol), "+v"(oh), "+v"(os));
+      Q6Run q;
+      __builtin_memcpy(&q.l1, wr + ol + 32, 16);
+      __builtin_memcpy(&q.h, wr + oh, 16);
+      ld8_u2(wr + os, q.sa, q.sb);
+      __builtin_memcpy(&q.l0, wr + ol, 16);
+      q.d = *reinterpret_cast<const uint16_t*>(wr + ob + KNJ_Q6K_D);
+      if (resid) rv = resid[row];
+      __builtin_amdgcn_sched_barrier(0);
+      acc = q6_run_dot(q, o, xv);
+    }
+    acc = group_sum<LPR>(acc);
     if (sub == 0 && row < n_out) {
       const float v = resid ? rv + acc : acc;
       y[row] = v;
@@ -589,8 +595,9 @@ bool bf16_fast(int n_in) {
 // Grids of the argmax-capable GEMVs (Q6_K, BF16, F32); one key per workgroup.
 int gemv_grid(int type, int n_in, int n_out) {
   if (type == KNJ_TYPE_Q6_K && n_in <= 4096) {
-    // three workgroups per CU, the rows walked grid-stride (the 151,936-row
-    // head: 52.4 us at 512, 47.5 at 768, 54.3 at 1024, 53.3 at 2048)
+    // three workgroups per CU, the rows walked grid-stride (151,936 x 2048 rows
+    // 52.0 us at 512 workgroups, 48.6 at 768, 50.1 at 1024, 50.4 at 2048; 32,768
+    // x 4096 25.5, 23.2, 24.3, 26.8; 12,000 x 2304 9.7, 9.2, 9.0, 10.6)
     const int rows = 4 * (64 / pow2_at_least(n_in / 64));  // of a workgroup's step
     return std::max(1, std::min(768, (n_out + rows - 1) / rows));
   }

@@ -30,20 +30,47 @@ def test_gemv_q6k_edges(device, n_in, n_out, fused):
         x64 = x64 / np.sqrt(np.mean(x64 * x64) + 1e-6) * nw
     wd = O.dequant(K.TYPE_Q6_K, w, n_in * n_out).astype(np.float64).reshape(n_out, n_in)
     want = wd @ x64 + (r if fused else 0.0)
-    blocks = np.ascontiguousarray(w).view(np.uint8).reshape(n_out, n_in // 256, 210)
-    d = np.ascontiguousarray(blocks[:, :, 208:210]).view(np.float16).astype(np.float64)
-    step = np.abs(np.ascontiguousarray(blocks[:, :, 192:208]).view(np.int8) * d)  # |d sc| per 16 weights
-    # The dot is d sc (sum q x - 32 sum x): terms up to |w| + 64 |d sc| in
-    # size, no chain of additions over 64 long on any route, a product each,
-    # and with the norm a few roundings more on x (its mean square's too).
-    size = (np.abs(wd) + 64.0 * np.repeat(step.reshape(n_out, -1), 16, axis=1)) @ np.abs(x64)
-    bound = 80 * U * (size + (np.abs(r) if fused else 0.0))
+    # Weights are exact in the sums' terms and no chain of additions is over 32
+    # long on any route; with the norm the roundings of x's mean square, its
+    # root and the two products come on top.
+    bound = (32 + 32 * fused) * U * (np.abs(wd) @ np.abs(x64) + (np.abs(r) if fused else 0.0))
     kw = dict(norm_w=K.DeviceBuffer.from_array(nw), eps=1e-6, resid=K.DeviceBuffer.from_array(r)) if fused else {}
     dy = K.DeviceBuffer(4 * n_out)
     K.gemv(K.TYPE_Q6_K, K.DeviceBuffer.from_array(w), n_in, n_out, K.DeviceBuffer.from_array(x), dy, **kw)
     got = dy.download(np.float32).astype(np.float64)
     assert np.all(np.abs(got - want) <= bound)
     assert rel_rmse(got, want) <= 1e-5
+
+
+@pytest.mark.parametrize("n_in", [256, 768, 2048, 2304, 4096, 4352])
+def test_gemv_q6k_lone_weights(device, n_in):
+    """Rows with one nonzero weight each, at every position of a super-block in
+    turn: the output is that weight's product alone, with nothing of the other
+    inputs' size in its error (codes are stored with an offset of 32, and an
+    offset subtracted only from the finished sums leaves their rounding)."""
+    print(f"gemv q6_k lone weights {n_in}", flush=True)
+    n_out, nb = 1024, n_in // 256
+    rng = np.random.default_rng(n_in)
+    w = O.synth_tensor(O.tensor_key(SEED, 0, "q", -1), K.TYPE_Q6_K, n_in, n_out)
+    blocks = np.ascontiguousarray(w).view(np.uint8).reshape(n_out, nb, 210).copy()
+    ql, qh = blocks[:, :, :128].copy(), blocks[:, :, 128:192].copy()
+    blocks[:, :, :128], blocks[:, :, 128:192] = 0x00, 0xAA  # code 32: weight 0
+    for j in range(n_out):
+        # weight i of block b: half h, quarter t, byte l of the quarter
+        b, i = int(rng.integers(nb)), (j * 7 + j // 256) % 256
+        h, t, l = i // 128, i % 128 // 32, i % 32
+        at, low = 64 * h + l + 32 * (t & 1), 0xF << (4 * (t >> 1))
+        blocks[j, b, at] = ql[j, b, at] & low
+        at, high = 32 * h + l, 3 << (2 * t)
+        blocks[j, b, 128 + at] = (0xAA & ~high & 0xFF) | (qh[j, b, at] & high)
+    w = blocks.reshape(-1)
+    wd = O.dequant(K.TYPE_Q6_K, w, n_in * n_out).astype(np.float64).reshape(n_out, n_in)
+    assert np.all(np.count_nonzero(wd, axis=1) <= 1) and np.count_nonzero(wd) > 0.9 * n_out
+    x = rng.standard_normal(n_in).astype(np.float32)
+    dy = K.DeviceBuffer(4 * n_out)
+    K.gemv(K.TYPE_Q6_K, K.DeviceBuffer.from_array(w), n_in, n_out, K.DeviceBuffer.from_array(x), dy)
+    got, want = dy.download(np.float32).astype(np.float64), wd @ x.astype(np.float64)
+    assert np.all(np.abs(got - want) <= 4 * U * np.abs(want))  # the code's, the scale's and d's product
 
 
 @pytest.mark.parametrize("n_embd,n_vocab,B", [(256, 65, 1), (512, 2049, 3), (1280, 4127, 33), (2048, 2048, 5)])
