@@ -703,8 +703,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
 // acc += d cq - dmin cm.  A comes straight from global memory (the pairs'
 // rows are shared by every workgroup of the expert and stay in L2).
 constexpr int kFew = 8;
-// the few kernels when pairs < kFewBelow * experts (measured crossover with
-// the 32-pair kernels: between 8 and 12 pairs per expert)
+// the few kernels when pairs < kFewBelow * experts (the crossover with the
+// 32-pair kernels lay between 8 and 12 pairs per expert with gate/up in
+// k_group_fewk)
 constexpr int kFewBelow = 10;
 
 __device__ __forceinline__ f32x4 mfma16(half8 a, half8 b, f32x4 c) {
@@ -795,15 +796,19 @@ __device__ __forceinline__ void few_superblock(const FewBlock& b, const half8 (&
   for (int i = 0; i < 4; ++i) acc[i] += d * cq[i] - dmin * cm[i];
 }
 
-// The few-pair down product with the reduction split over the waves of a
-// workgroup: workgroup = (FT 16-row tiles) x (up to 8 pairs of
-// one expert); wave w takes super-blocks w, w + KS, ... (KS = waves, NSBW per
-// wave) and issues every load of them before any arithmetic, so a workgroup
-// asks for whole rows (all super-blocks) of its tiles at once.  The waves'
-// partial tiles meet in LDS and are added in wave order.
-template <int FT, int NSBW>
+// The few-pair product with the reduction split over the waves of a workgroup
+// (the down product, and the gate/up product with SwiGLU where
+// few_gateup_units says so): workgroup = (FT 16-row tiles of every matrix) x
+// (up to 8 pairs of one expert); wave w takes super-blocks w, w + KS, ... (KS =
+// waves, NSBW per wave) and issues every load of them before any arithmetic, so
+// a workgroup asks for whole rows (all super-blocks) of its tiles at once.  The
+// waves' partial tiles meet in LDS and are added in wave order.
+template <bool GATEUP, int FT, int NSBW>
 __global__ __launch_bounds__(256) void k_group_fewk(GroupArgs a) {
-  __shared__ f32x4 part[4][FT][64];
+  static_assert(!GATEUP || FT == 2, "gate/up writes whole 32-row sub-blocks");
+  constexpr int NM = GATEUP ? 2 : 1;
+  __shared__ f32x4 part[4][NM * FT][64];
+  __shared__ float vs[GATEUP ? 32 : 1][kFew];  // the workgroup's gate/up outputs
   // (the plain order: the XCD-aware mapping of the 32-pair kernels measured
   // slower here, where an expert rarely has more than one item)
   const int item = blockIdx.y, rblock = blockIdx.x;
@@ -825,7 +830,7 @@ __global__ __launch_bounds__(256) void k_group_fewk(GroupArgs a) {
   const _Float16* sbase = (apart ? a.sl : a.sh) + (uint64_t)ap * 8 + 2 * kq;
   const FewLane L(kq);
   struct Buf {
-    FewBlock w[FT];
+    FewBlock w[NM][FT];
     half8 x[8];
     uint32_t s2;
   };
@@ -835,13 +840,16 @@ __global__ __launch_bounds__(256) void k_group_fewk(GroupArgs a) {
     const int sb = wave + KS * i;
     if (sb < nsb) {  // uniform over the wave
 #pragma unroll
-      for (int f = 0; f < FT; ++f) {
-        const int row = min(rbase + 16 * f + col, a.n_out - 1);
-        const uint8_t* p = a.w0 + (uint64_t)e * slab + (uint64_t)row * rb + (uint64_t)sb * KNJ_Q4K_BLOCK;
-        B[i].w[f].h = *reinterpret_cast<const uint4*>(p);
-        B[i].w[f].c0 = *reinterpret_cast<const uint4*>(p + KNJ_Q4K_QS + 32 * kq);
-        B[i].w[f].c1 = *reinterpret_cast<const uint4*>(p + KNJ_Q4K_QS + 32 * kq + 16);
-      }
+      for (int mtx = 0; mtx < NM; ++mtx)
+#pragma unroll
+        for (int f = 0; f < FT; ++f) {
+          const int row = min(rbase + 16 * f + col, a.n_out - 1);
+          const uint8_t* p = (mtx ? a.w1 : a.w0) + (uint64_t)e * slab + (uint64_t)row * rb +
+                             (uint64_t)sb * KNJ_Q4K_BLOCK;
+          B[i].w[mtx][f].h = *reinterpret_cast<const uint4*>(p);
+          B[i].w[mtx][f].c0 = *reinterpret_cast<const uint4*>(p + KNJ_Q4K_QS + 32 * kq);
+          B[i].w[mtx][f].c1 = *reinterpret_cast<const uint4*>(p + KNJ_Q4K_QS + 32 * kq + 16);
+        }
 #pragma unroll
       for (int u = 0; u < 8; ++u)
         B[i].x[u] = ld_h8(abase + (uint64_t)(32 * sb + 8 * kq + 4 * (u & 1) + (u >> 1)) * P * 8);
@@ -849,9 +857,11 @@ __global__ __launch_bounds__(256) void k_group_fewk(GroupArgs a) {
     }
   }
   __builtin_amdgcn_sched_barrier(0);
-  f32x4 acc[FT];
+  f32x4 acc[NM][FT];
 #pragma unroll
-  for (int f = 0; f < FT; ++f) acc[f] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int mtx = 0; mtx < NM; ++mtx)
+#pragma unroll
+    for (int f = 0; f < FT; ++f) acc[mtx][f] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int i = 0; i < NSBW; ++i) {
     if (wave + KS * i < nsb) {
@@ -859,23 +869,65 @@ __global__ __launch_bounds__(256) void k_group_fewk(GroupArgs a) {
       xm[0] = as_h2(B[i].s2).x;
       xm[1] = as_h2(B[i].s2).y;
 #pragma unroll
-      for (int f = 0; f < FT; ++f) few_superblock(B[i].w[f], B[i].x, xm, L, acc[f]);
+      for (int mtx = 0; mtx < NM; ++mtx)
+#pragma unroll
+        for (int f = 0; f < FT; ++f) few_superblock(B[i].w[mtx][f], B[i].x, xm, L, acc[mtx][f]);
     }
   }
 #pragma unroll
-  for (int f = 0; f < FT; ++f) part[wave][f][lane] = acc[f];
+  for (int mtx = 0; mtx < NM; ++mtx)
+#pragma unroll
+    for (int f = 0; f < FT; ++f) part[wave][mtx * FT + f][lane] = acc[mtx][f];
   __syncthreads();
-  // wave w finishes tiles w, w + KS, ..., the ranges added in wave order; lane's four values: pair 2 kq + i / 2, part i % 2, weight row
+  // wave w finishes tiles w, w + KS, ... of every matrix, the ranges added in
+  // wave order; lane's four values: pair 2 kq + i / 2, part i % 2, weight row
   // 16 f + col
   for (int f = wave; f < FT; f += KS) {
     const int row = rbase + 16 * f + col;
     if (row >= a.n_out) continue;
-    f32x4 s = part[0][f][lane];
-    for (int w = 1; w < KS; ++w) s += part[w][f][lane];
+    f32x4 s[NM];
+#pragma unroll
+    for (int mtx = 0; mtx < NM; ++mtx) {
+      s[mtx] = part[0][mtx * FT + f][lane];
+      for (int w = 1; w < KS; ++w) s[mtx] += part[w][mtx * FT + f][lane];
+    }
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int pj = 2 * kq + h;
-      if (pj < cnt) a.out[(uint64_t)(p0 + pj) * a.n_out + row] = s[2 * h] + s[2 * h + 1];
+      if (pj >= cnt) continue;
+      const float v = s[0][2 * h] + s[0][2 * h + 1];
+      if constexpr (GATEUP)
+        vs[16 * f + col][pj] = (v / (1.0f + expf(-v))) * (s[NM - 1][2 * h] + s[NM - 1][2 * h + 1]);
+      else
+        a.out[(uint64_t)(p0 + pj) * a.n_out + row] = v;
+    }
+  }
+  if constexpr (GATEUP) {
+    // the 32 rows [rbase, rbase + 32) of every pair in k_split_tile's layout:
+    // thread (pair pp, 8-group g) the group's high parts and remainders in
+    // perm8 order; per pair the 32-row sum, split the same way
+    __syncthreads();
+    const int t = threadIdx.x, pp = t & 7, g = t >> 3;
+    if (g < 4 && pp < cnt) {
+      half8 h, l;
+#pragma unroll
+      for (int jj = 0; jj < 8; ++jj) {
+        const float x = vs[8 * g + perm8(jj)][pp];
+        h[jj] = (_Float16)x;
+        l[jj] = (_Float16)(x - (float)h[jj]);
+      }
+      const uint64_t o = ((uint64_t)(rbase / 8 + g) * P + p0 + pp) * 8;
+      *reinterpret_cast<half8*>(a.oh + o) = h;
+      *reinterpret_cast<half8*>(a.ol + o) = l;
+    } else if (g == 4 && pp < cnt) {
+      float sum = 0.0f;
+#pragma unroll
+      for (int r = 0; r < 32; ++r) sum += vs[r][pp];
+      const _Float16 sh = (_Float16)sum;
+      const int b = rbase / 32;
+      const uint64_t o = ((uint64_t)(b / 8) * P + p0 + pp) * 8 + b % 8;
+      a.osh[o] = sh;
+      a.osl[o] = (_Float16)(sum - (float)sh);
     }
   }
 }
@@ -886,13 +938,15 @@ __global__ __launch_bounds__(256) void k_group_fewk(GroupArgs a) {
 // activations stay in registers for all units.  A unit's rows reach LDS by DMA
 // while the unit before it is decoded from there (two buffers, two workgroups
 // of eight waves per CU).  The waves' partial tiles meet in LDS and are added
-// in wave order by one of them.  The output is in k_split_tile's layout.
-// Bound by the decoding's vector instructions (about 120 per 16-row tile and
-// super-block, 36 matrix-core cycles per four of them): 616 pairs over 128
-// experts of 768 x 2048 take 61.8 us (226 MB of weights, 3.7 TB/s).  One
-// workgroup per 32 rows with every load before any arithmetic, which could
-// overlap the two only across workgroups, took 69 us; this kernel with four
-// waves of two super-blocks each 63-65 us.
+// in wave order by one of them while the others wait at the next unit's
+// barrier.  The output is in k_split_tile's layout.
+// Bound by the decoding's vector instructions (per 16-row tile and super-block
+// about 120, 480 issue cycles of a SIMD, against 144 cycles of its matrix core
+// for the nine products): 616 pairs over 128 experts of 768 x 2048 take 61.8 us
+// (226 MB of weights, 3.7 TB/s).  One workgroup per 32 rows with every load
+// before any arithmetic (k_group_fewk), which overlaps the two only across
+// workgroups, takes 69 us; this kernel with four waves of two super-blocks each
+// 63-65 us.
 //
 // A 16-row tile lies in LDS as groups of eight 16-byte pieces of every row (a
 // DMA instruction takes 128 contiguous bytes of eight rows); within its row's
@@ -1006,9 +1060,9 @@ __global__ __launch_bounds__(512, NSBW == 1 ? 4 : 2) void k_few_gateup(GroupArgs
     for (int mf = 0; mf < 2; ++mf)  // the products of the two parts of a pair's x together
       part[(wave * 2 + mf) * 64 + lane] = make_float2(acc[mf][0] + acc[mf][1], acc[mf][2] + acc[mf][3]);
     KNJ_FEW_BARRIER(kLdsOnly);
-    // one wave finishes the unit, the others go on to the next (the same wave
-    // for both units of 32 rows); lane's two values: pairs 2 kq and 2 kq + 1,
-    // weight row col
+    // one wave finishes the unit (the same wave for both units of 32 rows), the
+    // others wait for it at the next unit's barrier; lane's two values: pairs
+    // 2 kq and 2 kq + 1, weight row col
     if (wave != (u >> 1) % KS) continue;
     float2 g2 = part[lane], u2 = part[64 + lane];
     for (int w = 1; w < KS; ++w) {
@@ -1616,34 +1670,70 @@ hipError_t group_lds_attr() {
   return e;
 }
 
-// The few-pair gate/up product: KS = min(8, super-blocks) waves per workgroup.
+// The few-pair gate/up product in units: KS = min(8, super-blocks) waves per
+// workgroup.
 template <int NSBW>
-hipError_t launch_few_gateup_as(const GroupArgs& g, int max_items, hipStream_t s) {
+hipError_t launch_few_gateup_as(const GroupArgs& g, int units, int max_items, hipStream_t s) {
   static const hipError_t attr =
       hipFuncSetAttribute((const void*)k_few_gateup<NSBW>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 << 10);
   if (attr != hipSuccess) return attr;
   const int nsb = g.n_in >> 8, ks = std::min(8, nsb), ng = (9 * nsb + 7) / 8;
   const size_t lds = (size_t)(8 * ng + ks) << 10;  // two buffers of two tiles, the partial sums
-  // units per workgroup, an even number: more of them share the wait for the
-  // first, fewer fill the last round of workgroups (77 tokens / 32 sequences
-  // of the 768 x 2048 experts, whole layer and step: 117.9 us / 751 us with 4,
-  // 117.4 / 745 with 6, 119.8 / 745 with 8, 126.9 / 735 with 12, 120.2 / 785
-  // with 16)
-  const int units = 6;
   KNJ_LAUNCH(k_few_gateup<NSBW>, dim3((g.n_out / 16 + units - 1) / units, max_items), dim3(64 * ks), lds, s, g,
              units);
   return hipGetLastError();
 }
-hipError_t launch_few_gateup(const GroupArgs& g, int max_items, hipStream_t s) {
+template <int NSBW>
+hipError_t launch_fewk_gateup_as(const GroupArgs& g, int max_items, hipStream_t s) {
+  KNJ_LAUNCH((k_group_fewk<true, 2, NSBW>), dim3(g.n_out / 32, max_items), dim3(64 * std::min(4, g.n_in >> 8)), 0, s, g);
+  return hipGetLastError();
+}
+
+// Which form of the few-pair gate/up product: 0 for a workgroup per 32 rows
+// (k_group_fewk), else the units per workgroup of k_few_gateup (an even
+// number: more of them share the wait for the first, fewer fill the last round
+// of workgroups).  `items` is the number of work items to be expected.
+int few_gateup_units(int n_in, int n_out, double items) {
+  // rows of up to 1024: one super-block per wave, all of it in registers, four
+  // workgroups per CU (whole layer of 64 experts of 512 x 1024 over 1, 32 and
+  // 70 tokens: 28.0 / 40.2 / 44.7 us per 32 rows, 34.9 / 44.8 / 52.1 in units)
+  if (n_in <= 1024) return 0;
+  // lists that leave CUs idle in workgroups of six units, walked one after the
+  // other (128 experts of 768 x 2048, 1, 2 and 4 tokens = 62, 121 and 227
+  // workgroups: 33.8 / 39.4 / 48.9 us per 32 rows, 41.1 / 43.3 / 48.7 in units;
+  // 64 of 768 x 1792, 203 workgroups: 43.6 and 45.1; one workgroup per CU fits
+  // beyond 2048 inputs: 60 experts of 1280 x 3072, 106 and 198 workgroups:
+  // 48.1 / 65.3 and 49.2 / 59.0)
+  const double wgs = items * ((n_out / 16 + 5) / 6);
+  if (wgs < (n_in <= 2048 ? 212 : 112)) return 0;
+  // a second round of six units that would be less than about two thirds full:
+  // four (6 tokens of the 768 x 2048 experts = 321 workgroups 53.8 against 59.9
+  // us, 60 tokens of 256 x 2048 = 375 60.2 against 65.5; otherwise six is level
+  // or better: 32 and 150 tokens 87.4 against 89.3 and 154.9 against 156.2,
+  // eight and twelve lose up to 6 and 20 us)
+  return wgs > 256 && wgs <= 416 ? 4 : 6;
+}
+
+// The few-pair gate/up product.
+hipError_t launch_few_gateup(const GroupArgs& g, int n_expert, int max_items, hipStream_t s) {
   if (g.n_in % 256 || g.n_in <= 0 || g.n_in > 4096 || g.n_out % 32 || !g.oh) return hipErrorInvalidValue;
-  return g.n_in <= 8 * 256 ? launch_few_gateup_as<1>(g, max_items, s) : launch_few_gateup_as<2>(g, max_items, s);
+  // experts that P pairs reach when routing is even, or items of kFew full pairs
+  const double reach = n_expert * (1.0 - std::pow(1.0 - 1.0 / n_expert, g.P));
+  const int units = few_gateup_units(g.n_in, g.n_out, std::max(reach, (double)g.P / kFew));
+  if (units == 0) {
+    if (g.n_in <= 1024) return launch_fewk_gateup_as<1>(g, max_items, s);
+    if (g.n_in <= 2048) return launch_fewk_gateup_as<2>(g, max_items, s);
+    return launch_fewk_gateup_as<4>(g, max_items, s);
+  }
+  return g.n_in <= 8 * 256 ? launch_few_gateup_as<1>(g, units, max_items, s)
+                           : launch_few_gateup_as<2>(g, units, max_items, s);
 }
 
 // The few-pair down product: KS = min(4, super-blocks) waves per workgroup,
 // each with NSBW super-blocks of FT 16-row tiles.
 template <int FT, int NSBW>
 hipError_t launch_fewk_as(const GroupArgs& g, int max_items, hipStream_t s) {
-  KNJ_LAUNCH((k_group_fewk<FT, NSBW>), dim3((g.n_out + 16 * FT - 1) / (16 * FT), max_items),
+  KNJ_LAUNCH((k_group_fewk<false, FT, NSBW>), dim3((g.n_out + 16 * FT - 1) / (16 * FT), max_items),
              dim3(64 * std::min(4, g.n_in >> 8)), 0, s, g);
   return hipGetLastError();
 }
@@ -1714,7 +1804,7 @@ hipError_t launch_moe_batch(const MoeBatchArgs& a, void* scratch, hipStream_t s)
     gu.ol = al;
     gu.osh = sah;
     gu.osl = sal;
-    if (hipError_t e = launch_few_gateup(gu, max_items, s)) return e;
+    if (hipError_t e = launch_few_gateup(gu, E, max_items, s)) return e;
   } else {
     // SwiGLU written straight in the down product's operand layout
     gu.oh = ah;

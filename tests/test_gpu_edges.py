@@ -102,25 +102,29 @@ def test_batch_bf16_head_edges(device, n_embd, n_vocab, B):
     gm.close()
 
 
-@pytest.mark.parametrize("n_embd,n_ff,m", [(256, 256, 1), (768, 512, 9), (2304, 768, 5), (4096, 256, 12), (1024, 1280, 3)])
-def test_moe_few_pairs_edges(device, n_embd, n_ff, m):
+@pytest.mark.parametrize("n_embd,n_ff,n_expert,m", [
+    (256, 256, 8, 1), (768, 512, 8, 9), (2304, 768, 8, 5), (4096, 256, 8, 12), (1024, 1280, 8, 3),
+    (2048, 256, 8, 2), (1280, 256, 80, 120), (2304, 512, 32, 20), (1280, 1024, 32, 40)])
+def test_moe_few_pairs_edges(device, n_embd, n_ff, n_expert, m):
     """The few-pair expert products (fewer than ten pairs per expert) at one
     super-block, at counts of super-blocks that the waves of a workgroup share
-    unevenly, at the widest row, at row counts that leave the last workgroup a
-    remainder, and with items of one to eight pairs and more than one item per
-    expert: against the oracle within the parity bar (1e-5)."""
-    n_expert, k = 8, 4
-    print(f"few pairs {n_embd}x{n_ff} m={m}", flush=True)
+    unevenly, at the widest row, in each form of gate/up (32 rows at once for
+    narrow rows and short lists; six units with a last workgroup of four or two,
+    one and two super-blocks per wave; four units) and with items of one to
+    eight pairs: against the oracle within the parity bar (1e-5)."""
+    k = 4
+    print(f"few pairs {n_embd}x{n_ff} of {n_expert} m={m}", flush=True)
     syn = lambda kind, t, a, b, e=-1: O.synth_tensor(O.tensor_key(SEED, 1, kind, e), t, a, b)
     router = syn("router", K.TYPE_F32, n_embd, n_expert)
     gate, up = (np.concatenate([syn(n, K.TYPE_Q4_K, n_embd, n_ff, e) for e in range(n_expert)]) for n in ("gate", "up"))
     down = np.concatenate([syn("down", K.TYPE_Q4_K, n_ff, n_embd, e) for e in range(n_expert)])
     rng = np.random.default_rng(n_embd + m)
-    # (tokens 8 and later repeat the first: nine pairs and more on its experts)
     x = rng.standard_normal((m, n_embd)).astype(np.float32)
-    x[8:] = x[0]
+    if m >= 12:  # ten equal tokens: two work items for each of their experts
+        x[-9:] = x[0]
     resid = rng.standard_normal((m, n_embd)).astype(np.float32)
     want, _, ti_w, _ = O.moe(x, router, gate, up, down, n_embd, n_ff, n_expert, k, type_down=K.TYPE_Q4_K)
+    assert m < 12 or np.bincount(ti_w.ravel()).max() > 8
     d = [K.DeviceBuffer.from_array(a) for a in (x, router, gate, up, down)]
     out, logits = K.DeviceBuffer(4 * m * n_embd), K.DeviceBuffer(4 * m * n_expert)
     ti, tw = K.DeviceBuffer(4 * m * k), K.DeviceBuffer(4 * m * k)
