@@ -77,7 +77,8 @@ def test_gemv_q6k_lone_weights(device, n_in):
 def test_batch_bf16_head_edges(device, n_embd, n_vocab, B):
     """The batched bf16 head and its argmax at ragged row counts (64-row
     workgroups, 2048-entry argmax chunks), at one tile of sequences and more,
-    and at widths that leave the four K-splits uneven: logits against the
+    and at one to eight steps of 64 weights per wave (the model's widths are
+    multiples of 256, so the four waves' shares are equal): logits against the
     oracle's within the parity bar (1e-5), the greedy token exactly the batch's
     own first maximum."""
     print(f"batch head {n_embd}x{n_vocab} B={B}", flush=True)
@@ -133,3 +134,51 @@ def test_moe_few_pairs_edges(device, n_embd, n_ff, n_expert, m):
     got = out.download(np.float32).reshape(m, n_embd) - resid
     for t in range(m):
         assert rel_rmse(got[t], want[t]) <= 1e-5, t
+
+
+@pytest.mark.parametrize("n_head,n_kv,D", [(32, 4, 128), (16, 2, 64)])
+def test_decode_attention_long_cache(device, n_head, n_kv, D):
+    """The decode step's attention, which takes its position from the device and
+    so splits the whole cache's slots: one sequence and two in lockstep over
+    40,000 slots, seven and three chunks of 64 per workgroup, at positions that
+    leave the first split part-way, most splits past the position, one split
+    part-way far into the cache, and none.  The layer's output and the logits
+    against the oracle's over the same cache within the parity bar (1e-5)."""
+    n_ctx = 40000
+    print(f"decode attention {n_head}/{n_kv} x {D} over {n_ctx} slots", flush=True)
+    cfg = dict(n_layer=1, n_embd=512, n_head=n_head, n_head_kv=n_kv, head_dim=D, n_ff=256, n_expert=16,
+               n_expert_used=4, n_vocab=1024, n_ctx=n_ctx)
+    gm = K.Model.synthetic(K.qwen3_30b_a3b(**cfg), seed=SEED)
+    om = O.OracleModel(O.make_config(**cfg), seed=SEED, image=gm.download_image())
+    batch = K.Batch(gm, 2, n_ctx)
+    rng = np.random.default_rng(D)
+    shape = (1, n_kv, n_ctx, D)
+    kc = (0.7 * rng.standard_normal(shape, dtype=np.float32)).astype(np.float16).view(np.uint16)
+    vc = rng.standard_normal(shape, dtype=np.float32).astype(np.float16).view(np.uint16)
+    ok, ov = om.kv()
+
+    def same_as_oracle(tok, pos, cache, hidden, logits):
+        """The oracle's step over a cache that holds what the device appended."""
+        ok[...], ov[...] = kc, vc
+        om.set_kv_source(*cache)
+        om.set_pos(pos)
+        want = om.forward([tok])
+        assert om.kv_stats()["max_mid_dist"] <= 1e-5
+        assert rel_rmse(hidden, om.hidden(0)) <= 1e-5, pos
+        assert rel_rmse(logits, want) <= 1e-5, pos
+
+    for pos in (40, 160, 30100, n_ctx - 1):
+        print(f"position {pos}", flush=True)
+        gm.kv_upload(kc, vc)
+        gm.set_pos(pos)
+        lg = gm.forward([7])
+        same_as_oracle(7, pos, gm.kv_download(), gm.hidden(0), lg)
+        for s in range(2):
+            batch.kv_upload(s, kc, vc)
+        batch.set_pos(pos)
+        lg = batch.forward(np.array([7, 300], np.int32))
+        for s, tok in enumerate((7, 300)):
+            same_as_oracle(tok, pos, batch.kv_download(s), batch.hidden(0, s), lg[s])
+    batch.close()
+    om.close()
+    gm.close()
