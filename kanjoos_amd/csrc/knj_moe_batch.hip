@@ -351,7 +351,7 @@ struct GroupArgs {
   int P;                    // pairs
   const int4* items;        // {expert, first pair, pairs, 0}; null: dense, the P rows are one expert
   const int* n_items;
-  float* out;               // [pairs][n_out]
+  float* out;               // [pairs][n_out] (down and dense products)
   const float* resid = nullptr;  // optional [pairs][n_out] added to out (may alias out)
   // Split over the reduction (dense, not gate/up): blockIdx.z = k-range of
   // super-blocks [z * nsb / ksplit, (z + 1) * nsb / ksplit); with ksplit > 1
@@ -359,7 +359,6 @@ struct GroupArgs {
   // residual) and k_ksum adds the ranges in order.
   int ksplit = 1;
   float* partial = nullptr;
-  int tile = kTok;          // pairs per work item of the list (<= kTok)
   // gate/up: the output in k_split_tile's layout (f16 high parts, remainders,
   // per-32 sums)
   _Float16 *oh = nullptr, *ol = nullptr, *osh = nullptr, *osl = nullptr;
@@ -621,66 +620,63 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
   }
   __builtin_amdgcn_s_waitcnt(0);
   if constexpr (GATEUP) {
-    if (a.oh) {
-      // SwiGLU written straight as the down product's operand, the same
-      // values, order and roundings as k_split_tile over the f32 rows: the
-      // wave's 32 x 32 tile goes through its own LDS range (free after the
-      // last barrier) as [pair][row]; lane (pair, 8-group g of the wave's 32
-      // rows) then forms the perm8 high parts and remainders and the
-      // group's sequential sum, four consecutive lanes the 32-row sum
-      if (!rows_ok) return;
-      float* vs = reinterpret_cast<float*>(lds) + wave * 32 * 33;
+    // SwiGLU written straight as the down product's operand, the same
+    // values, order and roundings as k_split_tile over the f32 rows: the
+    // wave's 32 x 32 tile goes through its own LDS range (free after the
+    // last barrier) as [pair][row]; lane (pair, 8-group g of the wave's 32
+    // rows) then forms the perm8 high parts and remainders and the
+    // group's sequential sum, four consecutive lanes the 32-row sum
+    if (!rows_ok) return;
+    float* vs = reinterpret_cast<float*>(lds) + wave * 32 * 33;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int tj = 8 * (i / 4) + 4 * kh + (i % 4);
-        const float g = acc0[i];
-        vs[tj * 33 + j] = (g / (1.0f + expf(-g))) * acc1[i];
-      }
-      const int b = rbase >> 5;  // the 32-row sub-block of the wave
-#pragma unroll
-      for (int r = 0; r < 2; ++r) {
-        const int pr = 16 * r + (lane >> 2), g = lane & 3;
-        float v[8];
-#pragma unroll
-        for (int q = 0; q < 8; ++q) v[q] = vs[pr * 33 + 8 * g + q];
-        half8 h, l;
-        float sum = 0.0f;
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-          const float x = v[perm8(q)];
-          h[q] = (_Float16)x;
-          l[q] = (_Float16)(x - (float)h[q]);
-          sum += v[q];
-        }
-        sum = group_sum<4>(sum);
-        if (pr < cnt) {
-          const uint64_t o = ((uint64_t)((rbase >> 3) + g) * P + p0 + pr) * 8;
-          *reinterpret_cast<half8*>(a.oh + o) = h;
-          *reinterpret_cast<half8*>(a.ol + o) = l;
-          if (g == 0) {
-            const _Float16 sv = (_Float16)sum;
-            const uint64_t so = ((uint64_t)(b >> 3) * P + p0 + pr) * 8 + (b & 7);
-            a.osh[so] = sv;
-            a.osl[so] = (_Float16)(sum - (float)sv);
-          }
-        }
-      }
-      return;
+    for (int i = 0; i < 16; ++i) {
+      const int tj = 8 * (i / 4) + 4 * kh + (i % 4);
+      const float g = acc0[i];
+      vs[tj * 33 + j] = (g / (1.0f + expf(-g))) * acc1[i];
     }
-  }
-  if (!rows_ok || rbase + (lane & 31) >= a.n_out) return;
-  // acc[i] = C[token 8*(i/4) + 4*kh + i%4][row]
+    const int b = rbase >> 5;  // the 32-row sub-block of the wave
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int tj = 8 * (i / 4) + 4 * kh + (i % 4);
-    if (tj < cnt) {
-      float v = acc0[i];
-      if constexpr (GATEUP) v = (v / (1.0f + expf(-v))) * acc1[i];
-      const uint64_t o = (uint64_t)(p0 + tj) * a.n_out + row;
-      if (!GATEUP && a.ksplit > 1)
-        a.partial[(uint64_t)kz * P * a.n_out + o] = v;
-      else
-        a.out[o] = a.resid ? a.resid[o] + v : v;
+    for (int r = 0; r < 2; ++r) {
+      const int pr = 16 * r + (lane >> 2), g = lane & 3;
+      float v[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) v[q] = vs[pr * 33 + 8 * g + q];
+      half8 h, l;
+      float sum = 0.0f;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const float x = v[perm8(q)];
+        h[q] = (_Float16)x;
+        l[q] = (_Float16)(x - (float)h[q]);
+        sum += v[q];
+      }
+      sum = group_sum<4>(sum);
+      if (pr < cnt) {
+        const uint64_t o = ((uint64_t)((rbase >> 3) + g) * P + p0 + pr) * 8;
+        *reinterpret_cast<half8*>(a.oh + o) = h;
+        *reinterpret_cast<half8*>(a.ol + o) = l;
+        if (g == 0) {
+          const _Float16 sv = (_Float16)sum;
+          const uint64_t so = ((uint64_t)(b >> 3) * P + p0 + pr) * 8 + (b & 7);
+          a.osh[so] = sv;
+          a.osl[so] = (_Float16)(sum - (float)sv);
+        }
+      }
+    }
+  } else {
+    if (!rows_ok || rbase + (lane & 31) >= a.n_out) return;
+    // acc[i] = C[token 8*(i/4) + 4*kh + i%4][row]
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int tj = 8 * (i / 4) + 4 * kh + (i % 4);
+      if (tj < cnt) {
+        const float v = acc0[i];
+        const uint64_t o = (uint64_t)(p0 + tj) * a.n_out + row;
+        if (a.ksplit > 1)
+          a.partial[(uint64_t)kz * P * a.n_out + o] = v;
+        else
+          a.out[o] = a.resid ? a.resid[o] + v : v;
+      }
     }
   }
 }
@@ -1350,7 +1346,9 @@ __device__ __forceinline__ bf16x8 ld_b8(const uint16_t* p) {
 // them are in flight: 32 rows of 32,768 x 2048 took 70.6 us (1.9 TB/s) with a
 // workgroup of 128 rows, one wave per 32 rows and SIMD and no load ahead of
 // its use; 42.8 us (3.1 TB/s) with the K range over the waves, 64 rows per
-// activation load and a step of loads in flight.
+// activation load and a step's loads issued before the products of the step
+// before it (the copy at that step's end waits for them, so they are in flight
+// for those products only).
 constexpr int kBfRows = 64;
 
 struct Bf16Step {
@@ -1388,24 +1386,22 @@ __global__ __launch_bounds__(kBlock, 2) void k_dense_bf16(const uint16_t* __rest
   };
   f32x16 acc[2] = {};
   const int steps = n_in / 64;
-  if (wave < steps) {
-    Bf16Step cur, nxt;
-    load(wave, cur);
-    for (int st = wave; st < steps; st += 4) {
-      load(st + 4 < steps ? st + 4 : st, nxt);
-      // the loads stay ahead of the products (the scheduler would sink each to
-      // its use: 90 VGPRs, nothing in flight)
-      __builtin_amdgcn_sched_barrier(0);
+  Bf16Step cur, nxt;
+  load(wave, cur);
+  for (int st = wave; st < steps; st += 4) {
+    load(st + 4 < steps ? st + 4 : st, nxt);
+    // the loads stay ahead of the products (the scheduler would sink each to
+    // its use: 90 VGPRs, nothing in flight)
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
+    for (int u = 0; u < 4; ++u)
 #pragma unroll
-        for (int c = 0; c < 3; ++c)
+      for (int c = 0; c < 3; ++c)
 #pragma unroll
-          for (int t = 0; t < 2; ++t)
-            acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur.x[c][u], cur.w[t][u], acc[t], 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      cur = nxt;
-    }
+        for (int t = 0; t < 2; ++t)
+          acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur.x[c][u], cur.w[t][u], acc[t], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    cur = nxt;
   }
 #pragma unroll
   for (int t = 0; t < 2; ++t)
@@ -1642,7 +1638,6 @@ uint64_t moe_batch_scratch_bytes(int m, int n_embd, int n_ff, int n_expert, int 
   add(P * H / 16); add(P * H / 16);     // x sums hi/lo
   add(P * 4); add(P * 4);               // pair_tok, pair_of
   add(items * 16); add(256);            // items, n_items
-  add(P * F * 4);                       // act
   add(P * F * 2); add(P * F * 2);       // act hi/lo
   add(P * F / 16); add(P * F / 16);     // act sums hi/lo
   add(P * H * 4);                       // y
@@ -1774,7 +1769,6 @@ hipError_t launch_moe_batch(const MoeBatchArgs& a, void* scratch, hipStream_t s)
   int* pair_of = (int*)take(P * 4);
   int4* items = (int4*)take((uint64_t)max_items * 16);
   int* n_items = (int*)take(256);
-  float* act = (float*)take(P * F * 4);
   _Float16* ah = (_Float16*)take(P * F * 2);
   _Float16* al = (_Float16*)take(P * F * 2);
   _Float16* sah = (_Float16*)take(P * F / 16);
@@ -1796,26 +1790,19 @@ hipError_t launch_moe_batch(const MoeBatchArgs& a, void* scratch, hipStream_t s)
                      pair_of, items, n_items, tile);
   KNJ_LAUNCH(k_split_tile, dim3((unsigned)((P + 31) / 32), H / 64), dim3(kBlock), 0, s, xin,
              pair_tok, H, (int)P, xh, xl, sxh, sxl);
-  GroupArgs gu{a.gate, a.up, H, F, xh, xl, sxh, sxl, (int)P, items, n_items, act};
-  gu.tile = tile;
+  GroupArgs gu{a.gate, a.up, H, F, xh, xl, sxh, sxl, (int)P, items, n_items, nullptr};
+  // SwiGLU written straight in the down product's operand layout
+  gu.oh = ah;
+  gu.ol = al;
+  gu.osh = sah;
+  gu.osl = sal;
   if (few) {
-    // SwiGLU written straight in the down product's operand layout
-    gu.oh = ah;
-    gu.ol = al;
-    gu.osh = sah;
-    gu.osl = sal;
     if (hipError_t e = launch_few_gateup(gu, E, max_items, s)) return e;
   } else {
-    // SwiGLU written straight in the down product's operand layout
-    gu.oh = ah;
-    gu.ol = al;
-    gu.osh = sah;
-    gu.osl = sal;
     KNJ_LAUNCH(k_group_q4k<true>, dim3((F + kRowsWG - 1) / kRowsWG, max_items + 8), dim3(kBlock),
                kGroupLds, s, gu);
   }
   GroupArgs dn{a.down, nullptr, F, H, ah, al, sah, sal, (int)P, items, n_items, y};
-  dn.tile = tile;
   if (few && a.type_down == KNJ_TYPE_Q4_K) {
     if (hipError_t e = launch_fewk(dn, max_items, s)) return e;
   } else if (a.type_down == KNJ_TYPE_Q6_K)
@@ -1938,7 +1925,7 @@ hipError_t launch_dense_q4k_ex(const uint8_t* w, int n_in, int n_out, int m, con
 
 hipError_t launch_dense_bf16(const uint16_t* w, int n_in, int n_out, int m, const float* x,
                              float* out, void* scratch, hipStream_t s) {
-  if (n_in % 64) return hipErrorInvalidValue;
+  if (n_in % 256) return hipErrorInvalidValue;  // an equal share of 64-weight steps for each wave
   const uint64_t P = (uint64_t)m;
   uint8_t* p = (uint8_t*)scratch;
   auto take = [&](uint64_t bytes) {
