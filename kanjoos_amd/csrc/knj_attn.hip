@@ -12,6 +12,9 @@
 // only the workgroup that owns it writes it to the cache), and emits a partial
 // record {max, sum, sum a*v} per query head.  A second launch merges each
 // head's partials.
+#include <cstddef>
+#include <type_traits>
+
 #include "knj_common.h"
 #include "knj_dev.h"
 
@@ -177,13 +180,23 @@ constexpr int kLdsOnly = vm_lds_imm(63);
 // the first chunk's DMA (measured 1-3% faster per step than the chunk first).
 // With a RopeRow the step's RoPE row and position are kernel arguments (a
 // caller that holds them on the host needs no copy to the device); the row is
-// read by vector loads from the argument segment, where the argument lies at
-// the next 16-byte boundary behind the two before it.
-constexpr size_t kRopeRowOffset = (sizeof(AttnArgs) + sizeof(int) + 15) & ~(size_t)15;
-static_assert(alignof(RopeRow) == 16, "kernel argument layout");
+// read by vector loads from the argument segment, which holds the kernel's one
+// argument.
+struct AttnStep {
+  AttnArgs a;
+  int cpw;  // chunks per workgroup
+};
+struct AttnRowStep {
+  AttnArgs a;
+  int cpw;
+  RopeRow row;
+};
 
-template <int D, class... Row>
-__global__ __launch_bounds__(kBlock, 4) void k_attention(AttnArgs a, int cpw, Row... row) {  // 4 waves per SIMD: 128 VGPRs
+template <int D, class Step = AttnStep>
+__global__ __launch_bounds__(kBlock, 4) void k_attention(Step step) {  // 4 waves per SIMD: 128 VGPRs
+  constexpr bool kRow = std::is_same_v<Step, AttnRowStep>;
+  const AttnArgs& a = step.a;
+  const int cpw = step.cpw;
   constexpr int ROWH = D + 8;            // f16 elements per query LDS row (16-byte pad)
   constexpr int EROW = kChunk + 4;       // floats per score row
   constexpr int T = D / 4;               // threads per head for the q pass
@@ -213,9 +226,9 @@ __global__ __launch_bounds__(kBlock, 4) void k_attention(AttnArgs a, int cpw, Ro
   const float* kz = a.k + z * a.qkv_stride;
   const float* vz = a.v + z * a.qkv_stride;
   const float *rc, *rs;
-  if constexpr (sizeof...(Row) != 0) {
+  if constexpr (kRow) {
     rc = (const float*)((const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr() +
-                        kRopeRowOffset);
+                        offsetof(AttnRowStep, row.tab));
     rs = rc + D / 2;
   } else {
     rc = a.rope_cos + (uint64_t)z * a.rope_stride;
@@ -255,8 +268,8 @@ __global__ __launch_bounds__(kBlock, 4) void k_attention(AttnArgs a, int cpw, Ro
   // the position by a scalar load (asm: as a vector load, the compiler's wait
   // for it would also wait for the DMA issued before it)
   int pos;
-  if constexpr (sizeof...(Row) != 0)
-    pos = (row.pos, ...);
+  if constexpr (kRow)
+    pos = step.row.pos;
   else
     asm volatile("s_load_dword %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=s"(pos) : "s"(a.pos + z) : "memory");
   vm_wait7<2 * NI>(l_q, l_qn, l_k, l_v, l_kn, l_cs, l_sn);
@@ -948,11 +961,12 @@ hipError_t launch_attention(const AttnArgs& a, hipStream_t s, const RopeRow* row
   if (n_split > max_split) return hipErrorInvalidValue;
   const int z = std::max(1, a.n_seq);
   if (row && (z != 1 || row->pos < 0 || row->pos >= a.n_ctx)) return hipErrorInvalidValue;
+  const dim3 grid(a.n_head_kv, n_split, z);
   if (a.head_dim == 128) {
     if (row)
-      KNJ_LAUNCH((k_attention<128, RopeRow>), dim3(a.n_head_kv, n_split, z), dim3(kBlock), 0, s, a, cpw, *row);
+      KNJ_LAUNCH((k_attention<128, AttnRowStep>), grid, dim3(kBlock), 0, s, AttnRowStep{a, cpw, *row});
     else
-      KNJ_LAUNCH(k_attention<128>, dim3(a.n_head_kv, n_split, z), dim3(kBlock), 0, s, a, cpw);
+      KNJ_LAUNCH(k_attention<128>, grid, dim3(kBlock), 0, s, AttnStep{a, cpw});
     // up to 128 splits: 16 dims per workgroup, 16 parts of at most 8 splits
     // (the loads a part holds cost at short contexts)
     if (z == 1 && !a.split_hi && n_split <= 128)
@@ -963,9 +977,9 @@ hipError_t launch_attention(const AttnArgs& a, hipStream_t s, const RopeRow* row
       KNJ_LAUNCH(k_attn_merge_head<128>, dim3(a.n_head, z), dim3(kBlock), 0, s, a, n_split);
   } else if (a.head_dim == 64) {
     if (row)
-      KNJ_LAUNCH((k_attention<64, RopeRow>), dim3(a.n_head_kv, n_split, z), dim3(kBlock), 0, s, a, cpw, *row);
+      KNJ_LAUNCH((k_attention<64, AttnRowStep>), grid, dim3(kBlock), 0, s, AttnRowStep{a, cpw, *row});
     else
-      KNJ_LAUNCH(k_attention<64>, dim3(a.n_head_kv, n_split, z), dim3(kBlock), 0, s, a, cpw);
+      KNJ_LAUNCH(k_attention<64>, grid, dim3(kBlock), 0, s, AttnStep{a, cpw});
     if (z == 1 && !a.split_hi && n_split <= 128)
       KNJ_LAUNCH((k_attn_merge<64, 16, 32>), dim3(a.n_head * 2, z), dim3(kBlock), 0, s, a, n_split);
     else if (z == 1 && !a.split_hi && n_split <= 256)
