@@ -92,11 +92,6 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 
-// 32-bit LDS address of a pointer into shared memory
-__device__ __forceinline__ uint32_t lds_addr(const void* p) {
-  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
-}
-
 // Four f16 of a transposed LDS read (ds_read_b64_tr_b16).  Within each group
 // of 16 lanes, lane 4q + e receives element e of the 8-byte pieces addressed
 // by lanes q, 4 + q, 8 + q and 12 + q, in that order: a 4 x 16 block of a
@@ -116,14 +111,6 @@ __device__ __forceinline__ void lds_wait8(u32x2* v) {
   asm volatile("s_waitcnt lgkmcnt(0)"
                : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]));
 }
-// LDS DMA of 16 bytes per lane (global_load_lds_dwordx4) by asm: lane l's
-// 16 bytes from g land at LDS address base + 16 l (base wave-uniform).  The
-// compiler's wait placement treats every LDS access after a DMA it knows of
-// as aliasing it and waits for all of them; a kernel using this form waits
-// for its DMA itself (vmcnt; in-order) before the barriers that hand the
-// rows over, and the compiler's own counts only grow stricter by it.  M0 is
-// reserved to the compiler, which sets it right before each of its own uses
-// and keeps no value in it across this asm.
 // A 16-byte global load by asm (for loads that precede an asm DMA: the
 // caller waits for them with an explicit count, which the compiler's own
 // count, blind to the DMA, would set too deep), and that wait.
@@ -138,29 +125,9 @@ __device__ __forceinline__ void vm_wait7(f32x4& a, f32x4& b, f32x4& c, f32x4& d,
 }
 __device__ __forceinline__ float4 as_f4(f32x4 v) { return make_float4(v[0], v[1], v[2], v[3]); }
 
-__device__ __forceinline__ void dma16(const void* g, uint32_t base) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(g), "s"(base) : "memory");
-}
-
 __device__ __forceinline__ void lds_tie8(u32x2* v) {
   asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]));
 }
-
-// s_waitcnt immediates (gfx9 encoding): at most n vector memory operations
-// of this wave outstanding and every LDS access complete; LDS only
-constexpr int vm_lds_imm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4); }
-constexpr int kLdsOnly = vm_lds_imm(63);
-// Workgroup barrier after the wait `imm`.  __syncthreads() is a release fence
-// plus the barrier and the fence waits for every LDS DMA in flight, which
-// would drain the next chunk's fetch at every barrier of a chunk; the asm's
-// memory clobber keeps the compiler from moving memory accesses across it.
-#define KNJ_ATTN_BARRIER(imm)                 \
-  do {                                        \
-    __builtin_amdgcn_s_waitcnt(imm);          \
-    __builtin_amdgcn_sched_barrier(0);        \
-    asm volatile("s_barrier" ::: "memory");   \
-    __builtin_amdgcn_sched_barrier(0);        \
-  } while (0)
 
 // Decode attention of one new token per sequence: workgroup (kv head, split
 // of the KV range, sequence).  The G query heads of the kv head are
@@ -319,14 +286,14 @@ __global__ __launch_bounds__(kBlock, 4) void k_attention(Step step) {  // 4 wave
     const int cnt = min(kChunk, n_kv - p0);
     // 3) chunk j's K has landed (its V, fetched after it, may still be in
     // flight); the barrier also hands the query rows over on the first pass
-    KNJ_ATTN_BARRIER(vm_lds_imm(NI));
+    KNJ_BARRIER_AFTER(vm_lds_imm(NI));
     KNJ_STAMP(2);
     const bool here = pos >= p0 && pos < p0 + kChunk;  // uniform
     const int lp = pos - p0;
     if (here) {
       // the step's key replaces the fetched row (fetched before this step's write)
       if (tid < T) *reinterpret_cast<uint2*>(ks + lp * RB + 16 * kslot(lp, tid >> 1) + 8 * (tid & 1)) = kh2;
-      KNJ_ATTN_BARRIER(kLdsOnly);
+      KNJ_BARRIER_AFTER(kLdsOnly);
     }
     KNJ_STAMP(3);
     // 4) scores on the matrix cores: wave w computes S[p][h] for the 16 slots
@@ -353,7 +320,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_attention(Step step) {  // 4 wave
         for (int i = 0; i < 4; ++i) es[r * EROW + 16 * wave + 4 * kq + i] = sa[i] * scale2;
       }
     }
-    KNJ_ATTN_BARRIER(kLdsOnly);
+    KNJ_BARRIER_AFTER(kLdsOnly);
     // every wave's K reads are done: the next chunk's K
     if (j + 1 < nch) dma(p0 + kChunk, true, false);
     // 5) online softmax of the chunk: wave w owns heads 2w, 2w+1; lane = slot
@@ -391,15 +358,15 @@ __global__ __launch_bounds__(kBlock, 4) void k_attention(Step step) {  // 4 wave
       }
     }
     // chunk j's V has landed (the next chunk's K may stay in flight)
-    if (j + 1 < nch) KNJ_ATTN_BARRIER(vm_lds_imm(NI));
-    else KNJ_ATTN_BARRIER(vm_lds_imm(0));
+    if (j + 1 < nch) KNJ_BARRIER_AFTER(vm_lds_imm(NI));
+    else KNJ_BARRIER_AFTER(vm_lds_imm(0));
     if (here) {
       // the step's value replaces the fetched row, and the rows past it
       // become zeros (finite under their weight of 0)
       if (tid < T) *reinterpret_cast<uint2*>(vs + lp * RB + 16 * vslot(lp, tid >> 1) + 8 * (tid & 1)) = vh2;
       for (int o = (lp + 1) * RB + 16 * tid; o < CB; o += 16 * kBlock)
         *reinterpret_cast<uint4*>(vs + o) = make_uint4(0u, 0u, 0u, 0u);
-      KNJ_ATTN_BARRIER(kLdsOnly);
+      KNJ_BARRIER_AFTER(kLdsOnly);
     }
     KNJ_STAMP(4);
     // 6) sum e*v on the matrix cores: O[h][d] over the 64 slots.  Wave w owns
@@ -447,7 +414,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_attention(Step step) {  // 4 wave
       }
     }
     // every wave is done with V and es: the next chunk's V
-    KNJ_ATTN_BARRIER(kLdsOnly);
+    KNJ_BARRIER_AFTER(kLdsOnly);
     if (j + 1 < nch) dma(p0 + kChunk, false, true);
   }
   // 7) the step's row to the cache, by the workgroup that holds it

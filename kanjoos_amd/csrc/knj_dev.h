@@ -213,6 +213,43 @@ __device__ __forceinline__ bool last_block_done(unsigned int* counter, unsigned 
   return *flag_lds != 0u;
 }
 
+// ---- LDS DMA and waits counted by hand
+// s_waitcnt immediates (gfx9 encoding): at most n vector memory operations of
+// this wave outstanding and every LDS access of it complete; LDS only
+constexpr int vm_lds_imm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4); }
+constexpr int kLdsOnly = vm_lds_imm(63);
+
+// 32-bit LDS address of a pointer into shared memory
+__device__ __forceinline__ uint32_t lds_addr(const void* p) {
+  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
+}
+
+// LDS DMA of 16 bytes per lane (global_load_lds_dwordx4) by asm: lane l's
+// 16 bytes from g land at LDS address base + 16 l (base wave-uniform).  The
+// compiler's wait placement treats every LDS access after a DMA it knows of
+// as aliasing it and waits for all of them; a kernel using this form waits
+// for its DMA itself (vmcnt; in-order) before the barriers that hand the
+// rows over, and the compiler's own counts only grow stricter by it.  M0 is
+// reserved to the compiler, which sets it right before each of its own uses
+// and keeps no value in it across this asm.
+__device__ __forceinline__ void dma16(const void* g, uint32_t base) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(g), "s"(base) : "memory");
+}
+
+// Workgroup barrier after the wait `imm`.  __syncthreads() is a release fence
+// plus the barrier, and the fence waits for every outstanding load (LDS DMA
+// makes them count as LDS writes), which would empty a look-ahead at every
+// barrier; what a barrier hands over is covered by the explicit count instead.
+// The asm's memory clobber keeps the compiler from moving memory accesses
+// across it.
+#define KNJ_BARRIER_AFTER(imm)              \
+  do {                                      \
+    __builtin_amdgcn_s_waitcnt(imm);        \
+    __builtin_amdgcn_sched_barrier(0);      \
+    asm volatile("s_barrier" ::: "memory"); \
+    __builtin_amdgcn_sched_barrier(0);      \
+  } while (0)
+
 // Padded LDS layout of an activation vector: 16 bytes of padding after every 64
 // floats, so the 64-float slices that consecutive lanes read with ds_read_b128
 // start on different banks.

@@ -386,27 +386,6 @@ struct WBlock {
 typedef __attribute__((address_space(3))) void lds_void;
 typedef __attribute__((address_space(1))) void glb_void;
 
-// s_waitcnt immediate (gfx9 encoding) that waits until at most n vector
-// memory operations are outstanding and does not wait on the other counters
-constexpr int vmcnt_imm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
-// ... and that also waits for every LDS access of this wave
-constexpr int vm_lds_imm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4); }
-
-// Workgroup barrier once at most N vector memory operations of this wave
-// remain outstanding (and no LDS access).  __syncthreads() is a release fence
-// plus the barrier, and the fence waits for every outstanding load (the
-// LDS-DMA staging makes them count as LDS writes), which would empty the
-// weight look-ahead at every barrier; the staging a barrier hands over is
-// covered by the explicit count instead.  The asm's memory clobber keeps the
-// compiler from moving memory accesses across it.
-#define KNJ_BARRIER_VM(N)                      \
-  do {                                         \
-    __builtin_amdgcn_s_waitcnt(vm_lds_imm(N)); \
-    __builtin_amdgcn_sched_barrier(0);         \
-    asm volatile("s_barrier" ::: "memory");    \
-    __builtin_amdgcn_sched_barrier(0);         \
-  } while (0)
-
 // XCD-aware work mapping of a grouped launch (grid nrb row blocks x at least
 // 8 * ceil(n_items / 8) items): workgroups are dispatched to the eight XCDs
 // in turn by linear index, so XCD x runs linear indices x, x + 8, ...; this
@@ -501,9 +480,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
   if constexpr (NSBT > 1) {
     w_load(wr0, sbb + 1, w0s[1]);
     if constexpr (GATEUP) w_load(wr1, sbb + 1, w1s[1]);
-    KNJ_BARRIER_VM(WN);
+    KNJ_BARRIER_AFTER(vm_lds_imm(WN));
   } else {
-    KNJ_BARRIER_VM(0);
+    KNJ_BARRIER_AFTER(vm_lds_imm(0));
   }
   // super-block i on register set ci, the next weights into set ni
   auto step = [&](int i, int ci, int ni) __attribute__((always_inline)) {
@@ -601,9 +580,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
     // the staging done (at most the weight loads issued after it
     // outstanding) before the barrier that hands the buffer over
     if (load_next)
-      KNJ_BARRIER_VM(WN);
+      KNJ_BARRIER_AFTER(vm_lds_imm(WN));
     else
-      KNJ_BARRIER_VM(0);
+      KNJ_BARRIER_AFTER(vm_lds_imm(0));
   };
   if constexpr (NSBT > 0) {
 #pragma unroll
@@ -707,29 +686,6 @@ constexpr int kFewBelow = 10;
 __device__ __forceinline__ f32x4 mfma16(half8 a, half8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
 }
-
-
-// LDS DMA of 16 bytes per lane by asm, lane l's from g to LDS address
-// base + 16 l: the compiler's wait placement would make every LDS access after
-// a DMA that it knows of wait for it.  The kernel waits for its DMA itself
-// (vmcnt) before the barrier that hands the rows over; the compiler's own
-// counts only grow stricter by it.
-__device__ __forceinline__ uint32_t lds_addr(const void* p) {
-  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
-}
-__device__ __forceinline__ void dma16(const void* g, uint32_t base) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(g), "s"(base) : "memory");
-}
-constexpr int kLdsOnly = vm_lds_imm(63);
-// Workgroup barrier after the wait `imm` (__syncthreads() would wait for the
-// DMA in flight too).
-#define KNJ_FEW_BARRIER(imm)                \
-  do {                                      \
-    __builtin_amdgcn_s_waitcnt(imm);        \
-    __builtin_amdgcn_sched_barrier(0);      \
-    asm volatile("s_barrier" ::: "memory"); \
-    __builtin_amdgcn_sched_barrier(0);      \
-  } while (0)
 
 struct FewBlock {
   uint4 h, c0, c1;  // header (d, dmin, scales), the lane's 32 code bytes
@@ -1028,7 +984,7 @@ __global__ __launch_bounds__(512, NSBW == 1 ? 4 : 2) void k_few_gateup(GroupArgs
     const int buf = (u - u0) & 1;
     // the unit's rows have landed, every wave is past the buffer that the
     // next one fills
-    KNJ_FEW_BARRIER(vm_lds_imm(0));
+    KNJ_BARRIER_AFTER(vm_lds_imm(0));
     if (u + 1 < u1) fetch(u + 1, buf ^ 1);
     if (pend >= 0) store(pend);
     pend = -1;
@@ -1055,7 +1011,7 @@ __global__ __launch_bounds__(512, NSBW == 1 ? 4 : 2) void k_few_gateup(GroupArgs
 #pragma unroll
     for (int mf = 0; mf < 2; ++mf)  // the products of the two parts of a pair's x together
       part[(wave * 2 + mf) * 64 + lane] = make_float2(acc[mf][0] + acc[mf][1], acc[mf][2] + acc[mf][3]);
-    KNJ_FEW_BARRIER(kLdsOnly);
+    KNJ_BARRIER_AFTER(kLdsOnly);
     // one wave finishes the unit (the same wave for both units of 32 rows), the
     // others wait for it at the next unit's barrier; lane's two values: pairs
     // 2 kq and 2 kq + 1, weight row col
