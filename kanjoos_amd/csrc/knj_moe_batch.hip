@@ -578,7 +578,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
       for (int r = 0; r < 16; ++r) acc0[r] += d0 * (cqa[r] + cqb[r]) - m0 * cm0[r];
     }
     // the staging done (at most the weight loads issued after it
-    // outstanding) before the barrier that hands the buffer over
+    // outstanding) before the barrier that hands the buffer over.  (Unrolled,
+    // the weights stay in flight; in the any-range loop the compiler, which
+    // keeps no exact count across its back edge, waits for every load at the
+    // head of one of the two steps.)
     if (load_next)
       KNJ_BARRIER_AFTER(vm_lds_imm(WN));
     else
